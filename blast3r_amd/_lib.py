@@ -73,6 +73,10 @@ class BaPcgArgs(ctypes.Structure):
                 ('long_ptr', c_p), ('long_idx', c_p), ('img_part', c_p), ('src1', c_p), ('long_rng', c_p),
                 ('row_cap', c_int), ('real32', c_int)]
 
+class BaPcgPairs(ctypes.Structure):
+    _fields_ = [('t', c_p), ('p_img', c_p), ('up_ptr', c_p), ('n_pairs', c_i64)]
+
+
 class BaPmArgs(ctypes.Structure):
     _fields_ = [('infos', c_p), ('n_imgs', c_int), ('n_tracks', c_int),
                 ('run_ptr', c_p), ('run_obs', c_p), ('run_trk', c_p), ('run_img', c_p), ('img_run_ptr', c_p),
@@ -166,6 +170,8 @@ _SIGS = {
     'ba_pcg_solve': (c_int, [ctypes.POINTER(BaPcgArgs), c_p]),
     'ba_pcg_solve_range': (c_int, [ctypes.POINTER(BaPcgArgs), ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, c_p,
                                    c_p]),
+    'ba_pcg_solve_pairs_range': (c_int, [ctypes.POINTER(BaPcgArgs), ctypes.POINTER(BaPcgPairs), ctypes.c_int32,
+                                         ctypes.c_int32, ctypes.c_int32, c_p, c_p]),
     'ba_host_mapped_ptr': (c_p, [c_p]),
     'ba_pcg_partials_size': (c_i64, [c_i64]),
     'ba_apply_update': (c_int, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_f, c_f, c_int, c_int, c_int, c_int, c_i64,
@@ -204,7 +210,7 @@ EXPORTED = tuple(_SIGS)
 
 
 ABI_STRUCTS = {'ba_huber': BaHuber, 'ba_layout': BaLayout, 'ba_lin_args': BaLinArgs, 'ba_pm_args': BaPmArgs,
-               'ba_pcg_args': BaPcgArgs, 'ba_chol_args': BaCholArgs, 'ba_sample_args': BaSampleArgs,
+               'ba_pcg_args': BaPcgArgs, 'ba_pcg_pairs': BaPcgPairs, 'ba_chol_args': BaCholArgs, 'ba_sample_args': BaSampleArgs,
                'ba_obs_set': BaObsSet, 'ba_gather_args': BaGatherArgs, 'ba_remove_args': BaRemoveArgs,
                'ba_tangent_args': BaTangentArgs}
 

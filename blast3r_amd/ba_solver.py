@@ -83,6 +83,10 @@ def _flag(status, name, count, device):
     raise ValueError(f'bad {name}={status}')
 
 
+# Elements of the image-row copies above which the PCG's product goes by pair blocks (d <= 16): both measured on
+# retrieval structures, 300 iterations, with 10 M elements 1.9 us an iteration slower in fp64 and 0.6 us faster in
+# fp32, with 18 M 2.3 and 2.5 us faster, with 37 M 9.2 and 7.9 us, with 188 M 108 and 93 us
+PCG_ROWS_MOST = 14_000_000
 PCG_CHUNK = 25          # PCG iterations per graph when the host stops launching after the loop stops
 
 
@@ -503,8 +507,7 @@ class GaussNewtonSolver:
             self.last['direct'] = None
             direct_info = self._run_direct(pa, plan, st, n_imgs, um) if self.solver == 'cholesky' else None
             if direct_info is None:
-                self._pcg_rows(pa, plan, d, n_imgs)
-                self._run_pcg(pa, plan, st)
+                self._run_pcg(pa, self._pcg_rows(pa, plan, d, n_imgs), plan, st)
             self.last.update(rhs=rhs, diagA=diagA, damp=damp)
         else:
             direct_info = None
@@ -533,8 +536,7 @@ class GaussNewtonSolver:
         dX = backsubstitute()
         if direct_info is not None and not self._direct_status(direct_info):
             # a pivot was not positive: the device PCG solves the same system, then the points again
-            self._pcg_rows(pa, plan, d, n_imgs)
-            self._run_pcg(pa, plan, st)
+            self._run_pcg(pa, self._pcg_rows(pa, plan, d, n_imgs), plan, st)
             dX = backsubstitute()
         self.last.update(S_pairs=S_pairs, e_img=e_img, dg_img=dg_img, unknowns=um, lay=lay, plan=plan, x=x,
                          istate=istate, Hpp=Hpp, gp=gp, lam_p=lam_p, path=ctx['path'])
@@ -546,9 +548,11 @@ class GaussNewtonSolver:
 
     @staticmethod
     def _pcg_rows(pa, plan, d, n_imgs):
-        """The PCG's image-row copies of the pair blocks (workspace fields of ba_pcg_args), in the working
-        precision pa.real32 names."""
+        """The workspace of the PCG's products with S, in the working precision pa.real32 names: the image-row
+        copies of the pair blocks (fields of ba_pcg_args), or, where these would hold more than
+        PCG_ROWS_MOST elements, the arrays of the product by pair blocks (a ba_pcg_pairs, returned)."""
         ws = plan.workspace
+        R = torch.float32 if pa.real32 else torch.float64
         rp = plan.host['row_ptr']
         n_ent = int(rp[-1]) if len(rp) else 0
         # rows at a fixed capacity (the SpMV then needs no row_ptr load) when that pads by <= 25%
@@ -556,10 +560,15 @@ class GaussNewtonSolver:
         cap = -(-longest // 8) * 8
         row_cap = cap if 0 < cap and n_imgs * cap <= 1.25 * n_ent else 0
         n_blk = n_imgs * row_cap if row_cap else n_ent
-        S_rows = ws('pcg_S_rows', (max(n_blk, 1), d, d), torch.float32 if pa.real32 else torch.float64)
+        gw = 16 if d <= 16 else 32                     # lanes per block
+        if gw == 16 and n_blk * d * d > PCG_ROWS_MOST:
+            n_pairs = plan.scalars['n_pairs']
+            return _lib.BaPcgPairs(t=ptr(ws('pcg_t', (n_pairs, gw), R)), p_img=ptr(ws('pcg_p_img', (n_imgs, gw), R)),
+                                   up_ptr=ptr(ws('pcg_up_ptr', (n_imgs + 1,), torch.int32)), n_pairs=n_pairs)
+        S_rows = ws('pcg_S_rows', (max(n_blk, 1), d, d), R)
         pa.S_rows, pa.n_row_ent, pa.row_cap = ptr(S_rows), n_ent, row_cap
-        gw = 16 if d <= 16 else 32                     # row_u entries per block (the SpMV's lanes per group)
         pa.row_u = ptr(ws('pcg_row_u', (max(n_blk, 1) * gw,), torch.int32))
+        return None
 
     def _run_direct(self, pa, plan, st, n_imgs, um):
         """Enqueues ba_reduced_solve (L L^T of the damped reduced system, banded or dense) and returns
@@ -626,9 +635,9 @@ class GaussNewtonSolver:
             self.last['direct']['first_bad_pivot'] = bad
         return bad == 2 ** 31 - 1
 
-    def _run_pcg(self, pa, plan, st):
-        """ba_pcg_solve, replayed from HIP graphs captured once per argument set and kept with the plan.  The
-        iterations go in chunks of PCG_CHUNK, one graph each, whose last kernel stores the loop's stopped flag
+    def _run_pcg(self, pa, pw, plan, st):
+        """ba_pcg_solve (its product by pair blocks when pw is given), replayed from HIP graphs captured once per
+        argument set and kept with the plan.  The iterations go in chunks of PCG_CHUNK, one graph each, whose last kernel stores the loop's stopped flag
         to pinned host memory; the host reads chunk k's flag (after chunk k's event) while chunk k + 1 runs,
         and once the loop has stopped launches only the final decisions and the result (the reference checks
         its stopping rule after every iteration, bs:1216-1236).  The kernels skipped would have returned at
@@ -639,15 +648,15 @@ class GaussNewtonSolver:
         L = lib()
         self.last['pcg_launched'] = int(pa.maxiter)    # iterations launched (those after a stop return at once)
         if not self.use_graph:
-            check(L.ba_pcg_solve(pa, st))
+            check(self._pcg_range(pa, pw, 0, int(pa.maxiter), 1, None, st))
             return
         graphs = plan.__dict__.setdefault('_pcg_graphs', {})
-        key = bytes(pa)
+        key = bytes(pa) + (b'' if pw is None else bytes(pw))
         ent = graphs.get(key)
         if ent is None:
             if len(graphs) > 4:
                 graphs.clear()
-            ent = self._capture_pcg(pa)
+            ent = self._capture_pcg(pa, pw)
             graphs[key] = ent
         ent['solves'] += 1
         if ent['chunks'] is None or not (ent['early'] or ent['solves'] % 8 == 1):
@@ -672,7 +681,14 @@ class GaussNewtonSolver:
         self.last['pcg_launched'] = end
         ent['early'] = end < bounds[-1]
 
-    def _capture_pcg(self, pa):
+    @staticmethod
+    def _pcg_range(pa, pw, it0, it1, finish, stopped, st):
+        """ba_pcg_solve_range, or ba_pcg_solve_pairs_range when the product goes by pair blocks."""
+        if pw is None:
+            return lib().ba_pcg_solve_range(pa, it0, it1, finish, stopped, st)
+        return lib().ba_pcg_solve_pairs_range(pa, pw, it0, it1, finish, stopped, st)
+
+    def _capture_pcg(self, pa, pw):
         """The graphs of _run_pcg for one argument set: the whole sequence in one graph, and the iteration
         chunks (each storing its stopped flag) with the final decisions and result after each chunk."""
         L = lib()
@@ -688,13 +704,13 @@ class GaussNewtonSolver:
             with torch.cuda.graph(g):
                 check(fn(stream_ptr(dev)))
             return g
-        whole = capture(lambda s: L.ba_pcg_solve(pa, s))
+        whole = capture(lambda s: self._pcg_range(pa, pw, 0, maxit, 1, None, s))
         if not dptr:
             return dict(whole=whole, chunks=None, solves=0, early=False)
-        chunks = [capture(lambda s, k=k: L.ba_pcg_solve_range(pa, bounds[k], bounds[k + 1], 0,
-                                                               ctypes.c_void_p(dptr + 4 * k), s))
+        chunks = [capture(lambda s, k=k: self._pcg_range(pa, pw, bounds[k], bounds[k + 1], 0,
+                                                         ctypes.c_void_p(dptr + 4 * k), s))
                   for k in range(len(bounds) - 1)]
-        fin = {e: capture(lambda s, e=e: L.ba_pcg_solve_range(pa, e, e, 1, None, s)) for e in bounds[1:]}
+        fin = {e: capture(lambda s, e=e: self._pcg_range(pa, pw, e, e, 1, None, s)) for e in bounds[1:]}
         return dict(whole=whole, flags=flags, bounds=bounds, chunks=chunks, fin=fin, solves=0, early=False)
 
     def _add_z_prior(self, z_prior, lay, plan, S_pairs, e_img, dg_img):

@@ -483,6 +483,211 @@ __global__ void __launch_bounds__(PCG_T) k_pcg_update(ba_pcg_args a, int n) {
     if (threadIdx.x < PCG_NP) av.partials[PCG_NP * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? t[0] : t[1];
 }
 
+// ----------------------------------------------------------------------------- large systems
+// The product by pair blocks (d <= 16), for systems whose row copies would stream from memory on every
+// iteration: each block of the upper triangle is read once, in place in S_pairs, and serves both S x and
+// S^T x, where the row copies hold (and read) every off-diagonal block twice.  Bound by memory: at 4096 images,
+// 557 k pairs, d = 13 in fp64, k_pcg_pairs moves 0.82 GB in 179 us (4.6 TB/s, a large copy reaches 4.8), with
+// k_pcg_cols 21 us and k_pcg_dir 5 us, where k_pcg_spmv took 314 us for 1.5 GB; in fp32 93 us less an iteration.
+// The four launches of an iteration are
+//   k_pcg_dir(n)     the decisions after update n - 1 (as k_pcg_spmv forms them), p_n at image level
+//   k_pcg_pairs(n)   per image row its upper blocks: y_i, and t_p = S_p^T p_i per pair
+//   k_pcg_cols(n)    y_i += the t_p of the pairs whose second image is i; the row's share of p.Ap
+//   k_pcg_update(n)
+// Every sum runs in the order of the pair list.
+
+#define PCG_GW 16           // lanes per block, and the stride of t and p_img: whole 64- or 128-byte rows
+
+template <typename Real>
+struct PcgPairsV {
+    Real *t, *p_img;
+    const int32_t* up_ptr;
+    __device__ __forceinline__ explicit PcgPairsV(const ba_pcg_pairs& w)
+        : t((Real*)w.t), p_img((Real*)w.p_img), up_ptr(w.up_ptr) {}
+};
+
+// up_ptr[i] = the first pair of image row i (pair_i1 ascending), i = 0 .. n_imgs
+__global__ void __launch_bounds__(PCG_T) k_pcg_up_ptr(const int32_t* __restrict__ pair_i1, int64_t n_pairs, int n_imgs,
+                                                      int32_t* __restrict__ up_ptr) {
+    const int i = (int)(blockIdx.x * PCG_T + threadIdx.x);
+    if (i > n_imgs) return;
+    int64_t lo = 0, hi = n_pairs;
+    while (lo < hi) {
+        const int64_t m = (lo + hi) >> 1;
+        if (pair_i1[m] < i) lo = m + 1; else hi = m;
+    }
+    up_ptr[i] = (int32_t)lo;
+}
+
+// The decisions of k_pcg_spmv(n), from the same partial sums (every block forms them alike), the best-so-far
+// copy, and p_img[i][j] = p_n at entry (i, j) (0 past d and where the parameter is not an unknown).
+template <typename Real>
+__global__ void __launch_bounds__(PCG_T) k_pcg_dir(ba_pcg_args a, ba_pcg_pairs w, int n, int nb) {
+    const PcgV<Real> av(a);
+    const PcgPairsV<Real> pv(w);
+    __shared__ Real sh[2 * (PCG_T / 64)];
+    const int64_t e = (int64_t)blockIdx.x * PCG_T + threadIdx.x;
+    const int64_t i = e / PCG_GW;
+    const int j = (int)(e % PCG_GW), d = a.d;
+    const Real* __restrict__ pold = av.p + (int64_t)((n + 1) & 1) * a.n_u;
+    const Real best = av.state[ST_BEST0 + ((n - 1) & 1)], rz_old = av.state[ST_RZ0 + ((n - 1) & 1)];
+    const Real bnorm = av.state[ST_BNORM];
+    int u = -1;
+    Real zv = Real(0), po = Real(0);
+    if (i < a.n_imgs && j < d) {
+        u = a.umap[i * d + j];
+        if (u >= 0) { zv = av.z[u]; po = pold[u]; }
+    }
+    if (a.istate[IS_DONE0 + (n & 1)]) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.istate[IS_DONE0 + ((n + 1) & 1)] = 1;
+        return;
+    }
+    Real beta = Real(0);
+    if (n >= 1) {
+        Real rs[2];
+        sum_partials<PCG_T>(av.partials, nb, rs, sh);
+        const Real rnorm = sqrt(rs[0]), rz_new = rs[1];
+        const bool improved = rnorm < best;
+        const bool conv = rnorm <= Real(a.tol) * bnorm;
+        const bool bad = !isfinite(rz_new);
+        const bool stop = conv || bad || n >= a.maxiter;
+        beta = rz_new / (rz_old > Real(1e-32) ? rz_old : Real(1e-32));
+        if (improved)
+            for (int64_t v = e; v < a.n_u; v += (int64_t)gridDim.x * PCG_T) av.xbest[v] = av.x[v];
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            av.state[ST_BEST0 + (n & 1)] = improved ? rnorm : best;
+            if (improved) a.istate[IS_BESTK] = n;
+            av.state[ST_RZ0 + (n & 1)] = rz_new;
+            av.state[ST_BETA] = beta;
+            a.istate[IS_K] = n;
+            if (conv) { a.istate[IS_CONV] = 1; a.istate[IS_USEBEST] = 0; }
+            a.istate[IS_DONE0 + ((n + 1) & 1)] = stop;
+        }
+        if (stop) return;
+    } else if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.istate[IS_DONE0 + 1] = 0;
+    }
+    if (i < a.n_imgs) pv.p_img[e] = u >= 0 ? pdir(zv, po, beta) : Real(0);
+}
+
+// One workgroup per image row i, PCG_GW lanes per block, lane c holding column c of it: y_i[r] gathers
+// S[r][c] p_c per lane over the row's blocks (added over the lanes once per row), t_p[c] = sum_r S[r][c] p_i[r]
+// is the lane's own, so the loop needs no shuffles.  The next block's column is requested before this block's
+// products (three waves per SIMD in fp64; four, with spills, doubled the step's time).  Plain loads:
+// non-temporal ones cost 12%, and turning the row order round every other iteration for the memory-side cache
+// gained 0.5%.
+template <typename Real>
+__global__ void __launch_bounds__(PCG_T) k_pcg_pairs(ba_pcg_args a, ba_pcg_pairs w, int n) {
+    const PcgV<Real> av(a);
+    const PcgPairsV<Real> pv(w);
+    constexpr int NG = PCG_T / PCG_GW;
+    __shared__ Real sh[NG][PCG_GW];
+    const int i = blockIdx.x;
+    const int g = threadIdx.x / PCG_GW, c = threadIdx.x % PCG_GW;
+    const int d = a.d, dd = d * d;
+    if (a.istate[IS_DONE0 + ((n + 1) & 1)]) return;
+    const int p0 = pv.up_ptr[i], p1 = pv.up_ptr[i + 1];
+    Real xi[PCG_GW];                                      // p_n of this image (uniform over the workgroup)
+#pragma unroll
+    for (int r = 0; r < PCG_GW; ++r) xi[r] = pv.p_img[(int64_t)i * PCG_GW + r];
+    Real acc[PCG_GW];
+#pragma unroll
+    for (int r = 0; r < PCG_GW; ++r) acc[r] = Real(0);
+    auto load = [&](int p, Real& x, Real (&col)[PCG_GW]) {
+        const bool live = p < p1;
+        x = live ? pv.p_img[(int64_t)a.pair_i2[p] * PCG_GW + c] : Real(0);
+        const Real* S = av.S_pairs + (int64_t)p * dd + c;
+#pragma unroll
+        for (int r = 0; r < PCG_GW; ++r) col[r] = (live && c < d && r < d) ? S[r * d] : Real(0);
+    };
+    Real x, col[PCG_GW];
+    load(p0 + g, x, col);
+    for (int p = p0 + g; p < p1; p += NG) {
+        Real xn, coln[PCG_GW];
+        load(p + NG, xn, coln);
+        Real t = Real(0);
+#pragma unroll
+        for (int r = 0; r < PCG_GW; ++r) {
+            acc[r] = fma(col[r], x, acc[r]);
+            t = fma(col[r], xi[r], t);
+        }
+        pv.t[(int64_t)p * PCG_GW + c] = t;                // read by k_pcg_cols (never for a diagonal block)
+        x = xn;
+#pragma unroll
+        for (int r = 0; r < PCG_GW; ++r) col[r] = coln[r];
+    }
+    // sum of acc[r] over the group's lanes, left in lane r: each step halves the rows a lane keeps
+#pragma unroll
+    for (int h = PCG_GW / 2; h >= 1; h >>= 1) {
+        const bool up = (c & h) != 0;
+#pragma unroll
+        for (int r = 0; r < h; ++r) {
+            const Real send = up ? acc[r] : acc[r + h], keep = up ? acc[r + h] : acc[r];
+            acc[r] = keep + __shfl_xor(send, h, PCG_GW);
+        }
+    }
+    sh[g][c] = acc[0];
+    __syncthreads();
+    if (threadIdx.x < d) {
+        Real y = Real(0);
+        for (int k = 0; k < NG; ++k) y += sh[k][threadIdx.x];
+        av.y_img[(int64_t)i * d + threadIdx.x] = y;
+    }
+}
+
+// y_i += t_p over the pairs whose second image is i (the leading, transposed entries of its row list: the
+// pairs are ordered by first image), and the row's share of p.Ap: sum_e p_u(e) y_e plus the damping term of
+// the unknowns u = i + k n_imgs, as in k_pcg_spmv.
+template <typename Real>
+__global__ void __launch_bounds__(PCG_T) k_pcg_cols(ba_pcg_args a, ba_pcg_pairs w, int n) {
+    const PcgV<Real> av(a);
+    const PcgPairsV<Real> pv(w);
+    constexpr int NG = PCG_T / PCG_GW, NF = 4;            // entries in flight per group
+    __shared__ Real sh[NG][PCG_GW];
+    __shared__ Real sDamp[PCG_T / 64];
+    const int i = blockIdx.x;
+    const int g = threadIdx.x / PCG_GW, c = threadIdx.x % PCG_GW;
+    const int d = a.d;
+    const Real* __restrict__ pold = av.p + (int64_t)((n + 1) & 1) * a.n_u;
+    const Real beta = av.state[ST_BETA];
+    if (a.istate[IS_DONE0 + ((n + 1) & 1)]) return;
+    const int q0 = a.row_ptr[i], q1 = a.row_ptr[i + 1] - (pv.up_ptr[i + 1] - pv.up_ptr[i]);
+    Real y0 = Real(0), pi = Real(0);
+    if (threadIdx.x < d) { y0 = av.y_img[(int64_t)i * d + c]; pi = pv.p_img[(int64_t)i * PCG_GW + c]; }
+    Real acc = Real(0);
+    for (int q = q0 + g; q < q1; q += NG * NF) {
+        int ent[NF];
+#pragma unroll
+        for (int k = 0; k < NF; ++k) ent[k] = q + k * NG < q1 ? a.row_ent[q + k * NG] : -1;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) acc += ent[k] >= 0 ? pv.t[(int64_t)(ent[k] >> 1) * PCG_GW + c] : Real(0);
+    }
+    Real dsum = Real(0);
+    for (int64_t v = i + (int64_t)threadIdx.x * a.n_imgs; v < a.n_u; v += (int64_t)PCG_T * a.n_imgs) {
+        const Real pn = pdir(av.z[v], pold[v], beta);
+        dsum += av.damp[v] * pn * pn;
+    }
+    dsum = wave_sum(dsum);
+    sh[g][c] = acc;
+    if ((threadIdx.x & 63) == 0) sDamp[threadIdx.x >> 6] = dsum;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        Real part = Real(0);
+        if (threadIdx.x < d) {
+            Real y = y0;
+            for (int k = 0; k < NG; ++k) y += sh[k][c];
+            av.y_img[(int64_t)i * d + c] = y;
+            part = pi * y;
+        }
+        part = wave_sum(part);
+        if (threadIdx.x == 0) {
+#pragma unroll
+            for (int k = 0; k < PCG_T / 64; ++k) part += sDamp[k];
+            av.img_part[i] = part;
+        }
+    }
+}
+
 // the flag "stopped before update n" (read once the launches before it have run) to memory the host reads
 // (pinned host memory: a system-scope store)
 __global__ void k_pcg_stopped(const int32_t* __restrict__ flag, int32_t* out) {
@@ -525,43 +730,54 @@ int unknown_setup(const ba_pcg_args& a, hipStream_t st) {
 }
 }  // namespace ba
 
-// the launches of ba_pcg_solve_range in the working precision Real
-template <typename Real>
-static void pcg_launch(const ba_pcg_args& a, int32_t it0, int32_t it1, int32_t finish, int32_t* stopped_out,
-                       int64_t n_ent, unsigned nb, unsigned nbw, hipStream_t st) {
-    const int gw = a.d <= 16 ? 16 : 32;               // lanes per block row group of the SpMV (row_u stride)
+// the launches of ba_pcg_solve_range (w null) and ba_pcg_solve_pairs_range in the working precision Real, GW
+// lanes per block row
+template <int GW, typename Real>
+static void pcg_launch(const ba_pcg_args& a, const ba_pcg_pairs* w, int32_t it0, int32_t it1, int32_t finish,
+                       int32_t* stopped_out, int64_t n_ent, hipStream_t st) {
+    const unsigned nb = nb_of(a.n_u);
+    const unsigned nbw = (unsigned)((a.n_u + PCG_T / 64 - 1) / (PCG_T / 64));        // wave per unknown (setup)
     if (it0 == 0) {                                  // the setup precedes iteration 0
-        if (n_ent > 0)
+        if (w != nullptr)
+            hipLaunchKernelGGL(k_pcg_up_ptr, dim3(nb_of(a.n_imgs + 1)), dim3(PCG_T), 0, st, a.pair_i1, w->n_pairs,
+                               a.n_imgs, w->up_ptr);
+        else if (n_ent > 0)
             hipLaunchKernelGGL(k_rows_build<Real>, dim3((unsigned)((n_ent + PCG_T / 64 - 1) / (PCG_T / 64))),
-                               dim3(PCG_T), 0, st, a, n_ent, gw);
+                               dim3(PCG_T), 0, st, a, n_ent, GW);
         hipLaunchKernelGGL(k_unk_setup<Real>, dim3(nbw), dim3(PCG_T), 0, st, a);
         hipLaunchKernelGGL(k_leaf_max<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
         hipLaunchKernelGGL(k_leaf_damp<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
         hipLaunchKernelGGL(k_pcg_init<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
         hipLaunchKernelGGL(k_pcg_init2<Real>, dim3(1), dim3(PCG_T), 0, st, a, (int)nb);
     }
-    auto spmv = [&](int it) {
-        if (gw == 16)
-            hipLaunchKernelGGL((k_pcg_spmv<16, Real>), dim3((unsigned)a.n_imgs), dim3(PCG_ST), 0, st, a, it, (int)nb);
+    const dim3 rows((unsigned)a.n_imgs);
+    auto decide = [&](int it) {                      // the decisions after update it - 1, then p_it or A p_it
+        if (w != nullptr)
+            hipLaunchKernelGGL(k_pcg_dir<Real>, dim3(nb_of((int64_t)a.n_imgs * PCG_GW)), dim3(PCG_T), 0, st, a, *w, it,
+                               (int)nb);
         else
-            hipLaunchKernelGGL((k_pcg_spmv<32, Real>), dim3((unsigned)a.n_imgs), dim3(PCG_ST), 0, st, a, it, (int)nb);
+            hipLaunchKernelGGL((k_pcg_spmv<GW, Real>), rows, dim3(PCG_ST), 0, st, a, it, (int)nb);
     };
     for (int it = it0; it < it1; ++it) {
-        spmv(it);
+        decide(it);
+        if (w != nullptr) {
+            hipLaunchKernelGGL(k_pcg_pairs<Real>, rows, dim3(PCG_T), 0, st, a, *w, it);
+            hipLaunchKernelGGL(k_pcg_cols<Real>, rows, dim3(PCG_T), 0, st, a, *w, it);
+        }
         hipLaunchKernelGGL(k_pcg_update<Real>, dim3(nb), dim3(PCG_T), 0, st, a, it);
     }
     if (finish) {
         // the decisions after update it1 - 1 (after the last update, or a launch that returns at once once
         // the loop has stopped), then the result
-        spmv(it1);
+        decide(it1);
         hipLaunchKernelGGL(k_pcg_result<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
     } else if (stopped_out != nullptr) {
         hipLaunchKernelGGL(k_pcg_stopped, dim3(1), dim3(64), 0, st, a.istate + IS_DONE0 + (it1 & 1), stopped_out);
     }
 }
 
-extern "C" int ba_pcg_solve_range(const ba_pcg_args* args, int32_t it0, int32_t it1, int32_t finish,
-                                  int32_t* stopped_out, void* stream) {
+static int pcg_range(const ba_pcg_args* args, const ba_pcg_pairs* w, int32_t it0, int32_t it1, int32_t finish,
+                     int32_t* stopped_out, void* stream) {
     clear_error();
     BA_REQUIRE(args != nullptr, "null args");
     const ba_pcg_args& a = *args;
@@ -578,15 +794,39 @@ extern "C" int ba_pcg_solve_range(const ba_pcg_args* args, int32_t it0, int32_t 
                               a.y_img, a.partials, a.state, a.istate};
         for (const void* q : need) BA_REQUIRE(q != nullptr, "null pointer in ba_pcg_args");
     }
-    const unsigned nb = nb_of(a.n_u);
-    const unsigned nbw = (unsigned)((a.n_u + PCG_T / 64 - 1) / (PCG_T / 64));        // wave per unknown (setup)
-    BA_REQUIRE(a.row_cap >= 0 && a.row_cap % (PCG_ST / 16) == 0, "row_cap must be a multiple of 8");
-    const int64_t n_ent = a.row_cap > 0 ? (int64_t)a.n_imgs * a.row_cap : a.n_row_ent;
-    BA_REQUIRE(n_ent >= 0 && a.S_rows != nullptr && a.row_u != nullptr, "image-row block workspace missing");
-    if (a.real32) pcg_launch<float>(a, it0, it1, finish, stopped_out, n_ent, nb, nbw, st);
-    else          pcg_launch<double>(a, it0, it1, finish, stopped_out, n_ent, nb, nbw, st);
+    int64_t n_ent = 0;
+    if (w != nullptr) {
+        BA_REQUIRE(w->t != nullptr && w->p_img != nullptr && w->up_ptr != nullptr, "null pointer in ba_pcg_pairs");
+        BA_REQUIRE(a.d <= PCG_GW, "the product by pair blocks takes d <= 16");
+        BA_REQUIRE(w->n_pairs >= 0 && w->n_pairs < ((int64_t)1 << 30) && a.n_imgs >= 1, "bad pair or image count");
+    } else {
+        BA_REQUIRE(a.row_cap >= 0 && a.row_cap % (PCG_ST / 16) == 0, "row_cap must be a multiple of 8");
+        n_ent = a.row_cap > 0 ? (int64_t)a.n_imgs * a.row_cap : a.n_row_ent;
+        BA_REQUIRE(n_ent >= 0 && a.S_rows != nullptr && a.row_u != nullptr, "image-row block workspace missing");
+    }
+    if (a.d <= 16) {
+        if (a.real32) pcg_launch<16, float>(a, w, it0, it1, finish, stopped_out, n_ent, st);
+        else          pcg_launch<16, double>(a, w, it0, it1, finish, stopped_out, n_ent, st);
+    } else {
+        if (a.real32) pcg_launch<32, float>(a, w, it0, it1, finish, stopped_out, n_ent, st);
+        else          pcg_launch<32, double>(a, w, it0, it1, finish, stopped_out, n_ent, st);
+    }
     BA_LAUNCHED();
     return BA_OK;
+}
+
+extern "C" int ba_pcg_solve_range(const ba_pcg_args* args, int32_t it0, int32_t it1, int32_t finish,
+                                  int32_t* stopped_out, void* stream) {
+    return pcg_range(args, nullptr, it0, it1, finish, stopped_out, stream);
+}
+
+extern "C" int ba_pcg_solve_pairs_range(const ba_pcg_args* args, const ba_pcg_pairs* pairs, int32_t it0, int32_t it1,
+                                        int32_t finish, int32_t* stopped_out, void* stream) {
+    if (pairs == nullptr) {
+        clear_error();
+        BA_REQUIRE(false, "null pairs");
+    }
+    return pcg_range(args, pairs, it0, it1, finish, stopped_out, stream);
 }
 
 extern "C" int ba_pcg_solve(const ba_pcg_args* args, void* stream) {

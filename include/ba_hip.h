@@ -322,6 +322,19 @@ int ba_pcg_solve(const ba_pcg_args* args, void* stream);
  * system-scope store (pinned host memory).  ba_pcg_solve(a) = ba_pcg_solve_range(a, 0, maxiter, 1, NULL). */
 int ba_pcg_solve_range(const ba_pcg_args* args, int32_t it0, int32_t it1, int32_t finish, int32_t* stopped_out,
                        void* stream);
+/* The same solve with the product S p taken by pair blocks instead of by image-row copies: every block of the
+ * upper triangle is read once per iteration, in place in S_pairs, for S p and S^T p (four launches per
+ * iteration; half the bytes, for systems whose row copies do not stay in the caches); d <= 16.  S_rows, row_u, row_cap
+ * and n_row_ent of args are not used.  The pairs must be ordered by (pair_i1, pair_i2), i1 <= i2, and each
+ * image's row list must hold its pairs in pair order (as both planners make them). */
+typedef struct {
+    void* t;                           /* (R) (n_pairs, 16) workspace: S_p^T p per pair */
+    void* p_img;                       /* (R) (n_imgs, 16) workspace: p at image level */
+    int32_t* up_ptr;                   /* (n_imgs + 1) workspace: the first pair of each image row */
+    int64_t n_pairs;
+} ba_pcg_pairs;
+int ba_pcg_solve_pairs_range(const ba_pcg_args* args, const ba_pcg_pairs* pairs, int32_t it0, int32_t it1,
+                             int32_t finish, int32_t* stopped_out, void* stream);
 /* The device address of pinned, mapped host memory (hipPointerGetAttributes), or NULL when the device cannot
  * reach it: the stopped_out target of ba_pcg_solve_range (no counterpart in the reference). */
 void* ba_host_mapped_ptr(const void* host_ptr);
