@@ -77,6 +77,11 @@ class BaPcgPairs(ctypes.Structure):
     _fields_ = [('t', c_p), ('p_img', c_p), ('up_ptr', c_p), ('n_pairs', c_i64)]
 
 
+class BaPcgResident(ctypes.Structure):
+    _fields_ = [('words', c_p), ('shared_u', c_p), ('n_shared', c_int), ('m', c_int), ('max_blk', c_int),
+                ('max_col', c_int), ('limit', c_i64)]
+
+
 class BaPmArgs(ctypes.Structure):
     _fields_ = [('infos', c_p), ('n_imgs', c_int), ('n_tracks', c_int),
                 ('run_ptr', c_p), ('run_obs', c_p), ('run_trk', c_p), ('run_img', c_p), ('img_run_ptr', c_p),
@@ -172,6 +177,9 @@ _SIGS = {
                                    c_p]),
     'ba_pcg_solve_pairs_range': (c_int, [ctypes.POINTER(BaPcgArgs), ctypes.POINTER(BaPcgPairs), ctypes.c_int32,
                                          ctypes.c_int32, ctypes.c_int32, c_p, c_p]),
+    'ba_pcg_resident_plan': (ctypes.c_int32, [c_p, c_int, c_int, c_int, c_int, c_int, c_p, c_p]),
+    'ba_pcg_resident_words': (c_i64, [c_int, c_int, c_int, c_int]),
+    'ba_pcg_solve_resident': (c_int, [ctypes.POINTER(BaPcgArgs), ctypes.POINTER(BaPcgResident), c_p]),
     'ba_host_mapped_ptr': (c_p, [c_p]),
     'ba_pcg_partials_size': (c_i64, [c_i64]),
     'ba_apply_update': (c_int, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_f, c_f, c_int, c_int, c_int, c_int, c_i64,
@@ -210,7 +218,7 @@ EXPORTED = tuple(_SIGS)
 
 
 ABI_STRUCTS = {'ba_huber': BaHuber, 'ba_layout': BaLayout, 'ba_lin_args': BaLinArgs, 'ba_pm_args': BaPmArgs,
-               'ba_pcg_args': BaPcgArgs, 'ba_pcg_pairs': BaPcgPairs, 'ba_chol_args': BaCholArgs, 'ba_sample_args': BaSampleArgs,
+               'ba_pcg_args': BaPcgArgs, 'ba_pcg_pairs': BaPcgPairs, 'ba_pcg_resident': BaPcgResident, 'ba_chol_args': BaCholArgs, 'ba_sample_args': BaSampleArgs,
                'ba_obs_set': BaObsSet, 'ba_gather_args': BaGatherArgs, 'ba_remove_args': BaRemoveArgs,
                'ba_tangent_args': BaTangentArgs}
 

@@ -87,6 +87,7 @@ def _flag(status, name, count, device):
 # retrieval structures, 300 iterations, with 10 M elements 1.9 us an iteration slower in fp64 and 0.6 us faster in
 # fp32, with 18 M 2.3 and 2.5 us faster, with 37 M 9.2 and 7.9 us, with 188 M 108 and 93 us
 PCG_ROWS_MOST = 14_000_000
+RESIDENT_LIMIT = 10_000_000     # longest wait inside the resident solve, in ticks of 10 ns
 PCG_CHUNK = 25          # PCG iterations per graph when the host stops launching after the loop stops
 
 
@@ -506,11 +507,18 @@ class GaussNewtonSolver:
             pa.src1, pa.long_rng = ptr(um['src1']), ptr(um['long_rng'])
             self.last['direct'] = None
             direct_info = self._run_direct(pa, plan, st, n_imgs, um) if self.solver == 'cholesky' else None
-            if direct_info is None:
-                self._run_pcg(pa, self._pcg_rows(pa, plan, d, n_imgs), plan, st)
+            launches = lambda: self._run_pcg(pa, self._pcg_rows(pa, plan, d, n_imgs), plan, st)
+
+            def pcg():
+                """The device PCG, in one launch where that applies (returns True then)."""
+                if self._run_resident(pa, um, plan, st):
+                    return True
+                launches()
+                return False
+            resident = direct_info is None and pcg()
             self.last.update(rhs=rhs, diagA=diagA, damp=damp)
         else:
-            direct_info = None
+            direct_info, resident = None, False
         pm = ctx['path'] == 'pairmajor'
         has_X = en['X'][0] and (sc['n_runs'] > 0 if pm else sc['n_chunks'] > 0)
 
@@ -536,7 +544,10 @@ class GaussNewtonSolver:
         dX = backsubstitute()
         if direct_info is not None and not self._direct_status(direct_info):
             # a pivot was not positive: the device PCG solves the same system, then the points again
-            self._run_pcg(pa, self._pcg_rows(pa, plan, d, n_imgs), plan, st)
+            resident = pcg()
+            dX = backsubstitute()
+        if resident and not self._resident_status(istate, um, pa):
+            launches()                                 # the resident loop gave up waiting
             dX = backsubstitute()
         self.last.update(S_pairs=S_pairs, e_img=e_img, dg_img=dg_img, unknowns=um, lay=lay, plan=plan, x=x,
                          istate=istate, Hpp=Hpp, gp=gp, lam_p=lam_p, path=ctx['path'])
@@ -635,6 +646,41 @@ class GaussNewtonSolver:
             self.last['direct']['first_bad_pivot'] = bad
         return bad == 2 ** 31 - 1
 
+    def _run_resident(self, pa, um, plan, st):
+        """Enqueues ba_pcg_solve_resident (the whole loop in one launch) where it applies: rows that fit the
+        workgroups' registers and LDS, few shared unknowns, no capture under way, and no resident solve of this
+        structure that gave up waiting (as when another process holds part of the GPU).  Returns whether it was
+        launched; its outcome is read by _resident_status once the back-substitution is enqueued too."""
+        if pa.maxiter < 1 or torch.cuda.is_current_stream_capturing():
+            return False
+        sizes = um.get(('resident', pa.real32))
+        if sizes is None:
+            rp = np.ascontiguousarray(plan.host['row_ptr'][:pa.n_imgs + 1], dtype=np.int32)
+            blk, col = ctypes.c_int32(0), ctypes.c_int32(0)
+            n_cu = torch.cuda.get_device_properties(self.device).multi_processor_count
+            m = lib().ba_pcg_resident_plan(rp.ctypes.data_as(ctypes.c_void_p), pa.n_imgs, pa.d, pa.real32,
+                                           um['n_shared'], n_cu, ctypes.byref(blk), ctypes.byref(col))
+            sizes = um[('resident', pa.real32)] = (m, blk.value, col.value)
+        m, max_blk, max_col = sizes
+        if m < 1:
+            return False
+        L = lib()
+        nw = int(L.ba_pcg_resident_words(pa.n_imgs, pa.d, pa.real32, m))
+        pr = _lib.BaPcgResident(words=ptr(plan.workspace('pcg_words', (nw,), torch.int64)), shared_u=ptr(um['shared_u']),
+                                n_shared=um['n_shared'], m=m, max_blk=max_blk, max_col=max_col, limit=RESIDENT_LIMIT)
+        check(L.ba_pcg_solve_resident(pa, pr, st))
+        return True
+
+    def _resident_status(self, istate, um, pa):
+        """The resident solve's outcome (one read per solve): False when it gave up waiting, which keeps this
+        structure to the launch sequence from then on."""
+        ist = istate.tolist()
+        if ist[6]:
+            um[('resident', pa.real32)] = (0, 0, 0)
+            return False
+        self.last.update(pcg_launched=ist[2], pcg_resident=True)
+        return True
+
     def _run_pcg(self, pa, pw, plan, st):
         """ba_pcg_solve (its product by pair blocks when pw is given), replayed from HIP graphs captured once per
         argument set and kept with the plan.  The iterations go in chunks of PCG_CHUNK, one graph each, whose last kernel stores the loop's stopped flag
@@ -646,7 +692,8 @@ class GaussNewtonSolver:
         every eighth solve); so it is without a device-reachable flag, and launched directly with use_graph
         off."""
         L = lib()
-        self.last['pcg_launched'] = int(pa.maxiter)    # iterations launched (those after a stop return at once)
+        # iterations launched (those after a stop return at once)
+        self.last.update(pcg_launched=int(pa.maxiter), pcg_resident=False)
         if not self.use_graph:
             check(self._pcg_range(pa, pw, 0, int(pa.maxiter), 1, None, st))
             return

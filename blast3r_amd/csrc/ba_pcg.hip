@@ -9,6 +9,7 @@
 // _pcg line by line; scalars stay on the device (no host synchronisation).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 #include <cmath>
 
 #include "ba_common.h"
@@ -210,6 +211,7 @@ __global__ void __launch_bounds__(PCG_T) k_pcg_init2(ba_pcg_args a, int nb) {
         a.istate[IS_DONE0] = a.maxiter <= 0; a.istate[IS_DONE1] = 0; a.istate[IS_K] = 0; a.istate[IS_CONV] = 0;
         a.istate[IS_BESTK] = 0;
         a.istate[IS_USEBEST] = 1;
+        a.istate[6] = 0;                                       // set by a resident solve that gave up
     }
 }
 
@@ -688,6 +690,588 @@ __global__ void __launch_bounds__(PCG_T) k_pcg_cols(ba_pcg_args a, ba_pcg_pairs 
     }
 }
 
+// ----------------------------------------------------------------------------- resident solve
+// The whole loop in one cooperative launch, for systems whose image rows fit the workgroups' registers and LDS
+// and that share few unknowns.  A launch sequence pays two launches per iteration, and in each the dependent
+// loads of its operands; here every workgroup keeps m image rows (their blocks, the search direction at their
+// column images, the state of their unknowns) for the whole solve, and an iteration costs two exchanges:
+//   A  after update n - 1: each workgroup's partials of r.r and r.z, and z at its image-level entries
+//   B  after the product:  each workgroup's partials of p.Ap and of A p at the shared unknowns
+// Everything exchanged travels in words of eight bytes that hold 32 bits of data and the exchange's number, so
+// a reader that finds the number has the data: no fence, no barrier, no second load (a word is written once per
+// exchange, with a relaxed agent-scope store).  A word is overwritten only after its readers are done: what a
+// workgroup publishes in A follows its reading of B from every workgroup, each of which published B after it
+// had read A, and the other way round.
+// Every workgroup forms the loop's scalars from the same partials in the same order, so all decide alike.
+// A wait that exceeds its limit gives up: the workgroup sets istate[6] and leaves, the others follow, and the
+// caller solves by the launch sequence.
+// Bound by the exchanges' latency.  Per iteration, against the launch sequence (d = 13 where not said):
+//   1024 images, windows of 23, fp64 (205 workgroups)   10.3 us   15.3 us
+//   1024 images, the same, d = 9 (205)                   7.5 us   13.3 us
+//   256 images, 47 neighbours, fp64 (128)                8.1 us   15.0 us
+//   777 images, windows, fp32 (156)                      7.3 us   14.6 us
+//   500 images, d = 17, fp64 (167)                       8.5 us   18.2 us
+//   32 images, all pairs, fp32 (16)                      4.0 us   11.4 us
+//   8 images, fp64 (1, no exchange)                      2.0 us    7.1 us
+// of which (1024 images, cycles) A 6 to 7 k, B 9 k, the product 3.4 k, the updates and scalars 3 k.  While a
+// workgroup's own values are under way, its other waves stay at a barrier: polling then crowds out its stores.
+
+#define PP_T 512            // threads of a workgroup: PP_T / GW lane groups for the product
+#define PP_K 4              // column entries per thread
+#define PP_E 2              // own entries per lane of the first wave
+#define PP_NS 2             // most shared unknowns
+#define PP_G 16             // workgroups of a group whose partials its first one adds
+#define PP_WG 256           // most workgroups
+#define PP_LDS (158 * 1024) // dynamic LDS of a workgroup (160 KB per CU, less the static arrays)
+
+// {data, number} words of the exchanges: a double is two of them (low half, high half), a float one
+template <typename Real> struct LL;
+template <>
+struct LL<double> {
+    static constexpr int W = 2;
+    static __device__ __forceinline__ uint32_t part(double v, int h) {
+        return (uint32_t)(h ? __double2hiint(v) : __double2loint(v));
+    }
+    static __device__ __forceinline__ double join(const uint64_t (&w)[2]) {
+        return __hiloint2double((int)(uint32_t)w[1], (int)(uint32_t)w[0]);
+    }
+};
+template <>
+struct LL<float> {
+    static constexpr int W = 1;
+    static __device__ __forceinline__ uint32_t part(float v, int) { return __float_as_uint(v); }
+    static __device__ __forceinline__ float join(const uint64_t (&w)[1]) { return __uint_as_float((uint32_t)w[0]); }
+};
+__device__ __forceinline__ void ll_put(uint64_t* w, uint32_t data, uint32_t ep) {
+    __hip_atomic_store(w, (uint64_t)ep << 32 | data, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t ll_get(const uint64_t* w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One bounded wait of a thread: polls until try_() says that all its words have arrived, or the limit (ticks
+// of the 100 MHz clock) has passed; a limit of 0 gives up at once.
+template <typename F>
+__device__ __forceinline__ bool pp_wait(int64_t limit, F&& try_) {
+    int64_t t0 = 0;
+    for (unsigned k = 1;; ++k) {
+        if (limit <= 0) return false;
+        if (try_()) return true;
+        if ((k & 63) == 0) {
+            const int64_t t = (int64_t)wall_clock64();
+            if (k == 64) t0 = t;
+            else if (t - t0 > limit) return false;
+        }
+    }
+}
+
+// DPP move: lanes that have no source, or lie outside the row mask, get 0
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, true));
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp(double v) {
+    const long r = __builtin_amdgcn_update_dpp(0l, __builtin_bit_cast(long, v), CTRL, ROWS, 0xf, true);
+    return __builtin_bit_cast(double, r);
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// Sums over the wave without LDS (all lanes active): shifts within the rows of 16 lanes, then the rows' last
+// lanes into the rows above; every lane gets the total from lane 63.
+template <int K, typename Real>
+__device__ __forceinline__ void wave_sums(Real (&v)[K]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += dpp<0x111>(v[k]);              // row_shr:1
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += dpp<0x112>(v[k]);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += dpp<0x114>(v[k]);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += dpp<0x118>(v[k]);
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += dpp<0x142, 0xa>(v[k]);         // row_bcast:15
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += dpp<0x143, 0xc>(v[k]);         // row_bcast:31
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = lane_value(v[k], 63);
+}
+
+// num / den with inv = 1 / den at hand: the quotient corrected by its remainder
+template <typename Real>
+__device__ __forceinline__ Real div_by(Real num, Real den, Real inv) {
+    const Real q = num * inv;
+    return fma(fma(-q, den, num), inv, q);
+}
+
+// acc += sum over the columns c of a block of B[c][row] x[c], C0 <= c < DM, x[c] in lane c - C0 of the row of
+// 16 lanes (0 past d); the block's column c at the lane's row is col(c)
+template <int C0, int DM, int N = C0, typename Real, typename F>
+__device__ __forceinline__ void pp_cols(F&& col, Real x, Real (&acc)[2]) {
+    if constexpr (N < DM && N < C0 + 16) {
+        acc[N & 1] = fma(col(N), dpp<0x150 + N - C0>(x), acc[N & 1]);  // row_newbcast
+        pp_cols<C0, DM, N + 1>(col, x, acc);
+    }
+}
+
+// Blocks of a lane group that its lanes hold in registers (about 100 VGPRs of the 256 that two waves per SIMD
+// leave each); the others lie in LDS.
+constexpr int pp_regs_of(int dm, bool real32) {
+    return real32 ? (dm <= 16 ? 4 : dm <= 25 ? 3 : 2) : (dm <= 9 ? 3 : dm <= 16 ? 2 : dm <= 25 ? 1 : 0);
+}
+template <int DM, typename Real> struct PpRegs { static constexpr int N = pp_regs_of(DM, sizeof(Real) == 4); };
+// the unrolled block width: steps of about a quarter, so that little of an unrolled product is idle
+static inline int pp_width(int d) { return d <= 9 ? 9 : d <= 13 ? 13 : d <= 16 ? 16 : d <= 20 ? 20 : d <= 25 ? 25 : 32; }
+// An exchange of V partial sums per workgroup.  Up to 2 PP_G workgroups: each publishes its partials to
+// everyone (1.1 us).  More: to the first of its group of PP_G, which adds them (relay) and publishes the group's: every
+// workgroup polling the partials of 205 others took 3.5 to 4 us, two hops over few lines 2.8.  What everyone polls is
+// kept in as many copies as one store instruction writes, the readers spread over them, as the readers of one line
+// are served one after the other.
+template <int V, typename Real>
+struct PpSums {
+    typedef LL<Real> L;
+    static constexpr int W = L::W, VW = V * W, NC = 64 / VW;            // words of one publication; copies
+    uint64_t *xm, *xg;                                                  // to the group's first; to everyone
+    int nwg, wg, ng, gs;                                                // groups (padded to lines: gs)
+    bool two;
+    __device__ __forceinline__ PpSums(uint64_t* words, int nwg_, int wg_) : nwg(nwg_), wg(wg_) {
+        two = nwg > 2 * PP_G;
+        ng = two ? (nwg + PP_G - 1) / PP_G : nwg;
+        gs = (ng + 15) & ~15;
+        xg = words;
+        xm = words + (int64_t)64 * gs;
+    }
+    static __host__ __device__ int64_t words_of(int nwg) {
+        const int ng = nwg > 2 * PP_G ? (nwg + PP_G - 1) / PP_G : nwg;
+        return 64 * (int64_t)((ng + 15) & ~15) + (int64_t)(nwg + PP_G - 1) / PP_G * PP_G * 6;   // for every V <= 3
+    }
+    __device__ __forceinline__ int64_t words() const { return words_of(nwg); }
+    __device__ __forceinline__ Real pick(const Real (&v)[V], int s) const {
+        Real r = v[0];
+#pragma unroll
+        for (int k = 1; k < V; ++k) r = s == k ? v[k] : r;
+        return r;
+    }
+    // to everyone, as group g: lane l writes word l % VW of copy l / VW
+    __device__ __forceinline__ void put_all(const Real (&v)[V], uint32_t ep, int lane, int g) const {
+        const int c = lane % VW;
+        if (lane < NC * VW) ll_put(xg + lane * gs + g, L::part(pick(v, c / W), c % W), ep);
+    }
+    // one wave, all lanes holding the workgroup's partials
+    __device__ __forceinline__ void put(const Real (&v)[V], uint32_t ep, int lane) const {
+        if (!two) put_all(v, ep, lane, wg);
+        else if (lane < VW)
+            ll_put(xm + ((wg / PP_G) * VW + lane) * PP_G + wg % PP_G, L::part(pick(v, lane / W), lane % W), ep);
+    }
+    // the group's first workgroup, one wave: lane (value, member) polls one partial; the rows of 16 lanes are
+    // added and published
+    __device__ __forceinline__ bool relay(int64_t limit, uint32_t ep, int lane) const {
+        if (!two || wg % PP_G != 0) return true;
+        const int g = wg / PP_G, s = lane / 16, k = lane % 16;
+        Real x = Real(0);
+        bool good = true;
+        if (s < V && wg + k < nwg) {
+            const uint64_t* q = xm + (g * VW + s * W) * PP_G + k;
+            good = pp_wait(limit, [&]() {
+                uint64_t raw[W];
+                bool all = true;
+#pragma unroll
+                for (int h = 0; h < W; ++h) raw[h] = ll_get(q + h * PP_G);
+#pragma unroll
+                for (int h = 0; h < W; ++h) all = all && (uint32_t)(raw[h] >> 32) == ep;
+                x = L::join(raw);
+                return all;
+            });
+        }
+        x += dpp<0x111>(x);
+        x += dpp<0x112>(x);
+        x += dpp<0x114>(x);
+        x += dpp<0x118>(x);                                             // lane 15 of each row: its sum
+        Real v[V];
+#pragma unroll
+        for (int q = 0; q < V; ++q) v[q] = lane_value(x, 16 * q + 15);
+        put_all(v, ep, lane, g);
+        return good;
+    }
+    // one wave: lane g gets the partials of group g (0 past the groups); wave_sums makes the sums of them
+    __device__ __forceinline__ bool get(int64_t limit, uint32_t ep, int lane, Real (&v)[V]) const {
+#pragma unroll
+        for (int q = 0; q < V; ++q) v[q] = Real(0);
+        if (lane >= ng) return true;
+        const uint64_t* q = xg + (wg % NC) * VW * gs + lane;
+        return pp_wait(limit, [&]() {
+            uint64_t raw[V][W];
+            bool all = true;
+#pragma unroll
+            for (int s = 0; s < V; ++s)
+#pragma unroll
+                for (int h = 0; h < W; ++h) raw[s][h] = ll_get(q + (s * W + h) * gs);
+#pragma unroll
+            for (int s = 0; s < V; ++s) {
+#pragma unroll
+                for (int h = 0; h < W; ++h) all = all && (uint32_t)(raw[s][h] >> 32) == ep;
+                v[s] = L::join(raw[s]);
+            }
+            return all;
+        });
+    }
+};
+
+// LDS of a workgroup: the blocks of its rows that are not in registers (before they are loaded, the map from
+// images to column slots), then p at its column images, the lane groups' products, the column images and the
+// LDS blocks' column slots.
+struct PpLds {
+    size_t S, pcol, yp, col, cidx, total;
+};
+static __host__ __device__ inline PpLds pp_lds(int d, int gw, size_t R, int n_imgs, int max_blk, int max_col) {
+    PpLds o;
+    size_t at = 0;
+    auto take = [&](size_t n) { const size_t r = at; at += (n + 15) & ~(size_t)15; return r; };
+    const size_t sb = R * d * d * (size_t)max_blk, mb = sizeof(uint16_t) * (size_t)n_imgs;
+    o.S = take(sb > mb ? sb : mb);
+    o.pcol = take(R * gw * (size_t)max_col);
+    o.yp = take(R * PP_T);
+    o.col = take(sizeof(int) * (size_t)max_col);
+    o.cidx = take(sizeof(int) * (size_t)max_blk);
+    o.total = at;
+    return o;
+}
+
+__global__ void __launch_bounds__(PCG_T) k_pp_clear(uint64_t* __restrict__ w, int64_t n, int32_t* __restrict__ istate) {
+    const int64_t t = (int64_t)blockIdx.x * PCG_T + threadIdx.x;
+    if (t < n) w[t] = 0;
+    if (t < 8) istate[t] = 0;
+}
+
+// DM: the block width the product is unrolled for (d <= DM <= GW); NS: shared unknowns exchanged.  The first
+// wave owns the workgroup's entries (their x, r, z, p and the loop's partial sums); all waves poll, form the
+// loop's scalars and take part in the product.  Four barriers per iteration.
+template <int GW, int DM, int NS, typename Real>
+__global__ void __launch_bounds__(PP_T) k_pcg_resident(ba_pcg_args a, ba_pcg_resident w) {
+    typedef LL<Real> L;
+    constexpr int W = L::W, NG = PP_T / GW, NW = PP_T / 64;
+    extern __shared__ __align__(16) char lds[];
+    __shared__ Real sA[2];
+    __shared__ int sCnt[NW], sFailA, sFailB;
+    const PcgV<Real> av(a);
+    const int d = a.d, dd = d * d, tid = threadIdx.x, wg = blockIdx.x, nwg = gridDim.x, m = w.m;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const PpLds o = pp_lds(d, GW, sizeof(Real), a.n_imgs, w.max_blk, w.max_col);
+    Real* const sS = reinterpret_cast<Real*>(lds + o.S);
+    Real* const sP = reinterpret_cast<Real*>(lds + o.pcol);
+    Real* const sY = reinterpret_cast<Real*>(lds + o.yp);
+    int* const sCol = reinterpret_cast<int*>(lds + o.col);
+    int* const sCidx = reinterpret_cast<int*>(lds + o.cidx);
+    // word h of z at entry (i, j): xz[(i W + h) GW + j]
+    uint64_t* const xz = w.words;
+    const PpSums<2, Real> xA(w.words + (int64_t)a.n_imgs * GW * W, nwg, wg);
+    const PpSums<1 + NS, Real> xB(w.words + (int64_t)a.n_imgs * GW * W + xA.words(), nwg, wg);
+    const int i0 = wg * m, i1 = min(i0 + m, a.n_imgs);
+    const int e0 = a.row_ptr[i0], nblk = a.row_ptr[i1] - e0;
+    constexpr int NBR = PpRegs<DM, Real>::N;
+    if (tid == 0) { sFailA = 0; sFailB = 0; }
+
+    // ---- column images of the own rows: marked in a map, then numbered in image order
+    uint16_t* const map = reinterpret_cast<uint16_t*>(lds + o.S);
+    for (int i = tid; i < a.n_imgs; i += PP_T) map[i] = 0;
+    __syncthreads();
+    auto col_of = [&](int b) {
+        const int ent = a.row_ent[e0 + b], p = ent >> 1;
+        return (ent & 1) ? a.pair_i1[p] : a.pair_i2[p];
+    };
+    for (int b = tid; b < nblk; b += PP_T) map[col_of(b)] = 1;          // equal stores may meet
+    for (int i = i0 + tid; i < i1; i += PP_T) map[i] = 1;               // an own image without blocks, too
+    __syncthreads();
+    const int per = (a.n_imgs + PP_T - 1) / PP_T, lo = min(tid * per, a.n_imgs), hi = min(lo + per, a.n_imgs);
+    int cnt = 0;
+    for (int i = lo; i < hi; ++i) cnt += map[i];
+    int scan = cnt;                                                     // inclusive over the wave, then the waves
+    for (int s = 1; s < 64; s <<= 1) {
+        const int v = __shfl_up(scan, s);
+        if (lane >= s) scan += v;
+    }
+    if (lane == 63) sCnt[wave] = scan;
+    __syncthreads();
+    int base = scan - cnt, ncol = 0;
+    for (int k = 0; k < NW; ++k) {
+        if (k < wave) base += sCnt[k];
+        ncol += sCnt[k];                                                // at most max_col
+    }
+    for (int i = lo; i < hi; ++i)
+        if (map[i]) { map[i] = (uint16_t)base; sCol[base++] = i; }
+    __syncthreads();
+    // ---- the own entries, in the first wave: lane l holds entries l and l + 64 (entry e: image i0 + e / d,
+    // parameter e % d); an unknown shared by several entries has its state at each of them, and counts once (at
+    // the first entry of its list)
+    int u[PP_E], sh[PP_E], oy[PP_E], op[PP_E], ow[PP_E];
+    bool counts[PP_E];
+    Real x[PP_E], xb_[PP_E], r[PP_E], z[PP_E], p[PP_E], dA[PP_E], iA[PP_E], dmp[PP_E];
+    const int gpr = NG / m;                                             // lane groups per row
+#pragma unroll
+    for (int k = 0; k < PP_E; ++k) {
+        const int e = lane + 64 * k, el = e / d, ej = e - el * d;
+        u[k] = -1; sh[k] = -1; counts[k] = false;
+        oy[k] = op[k] = ow[k] = 0;
+        x[k] = xb_[k] = r[k] = z[k] = p[k] = dmp[k] = Real(0);
+        dA[k] = iA[k] = Real(1);
+        if (wave == 0 && e < (i1 - i0) * d) {
+            u[k] = a.umap[(int64_t)(i0 + el) * d + ej];
+            oy[k] = el * gpr * GW + ej;                                 // its products in sY
+            op[k] = map[i0 + el] * GW + ej;                             // its place in sP
+            ow[k] = ((i0 + el) * W) * GW + ej;                          // its words
+            if (u[k] >= 0) {
+                r[k] = av.rhs[u[k]]; dA[k] = av.diagA[u[k]]; dmp[k] = av.damp[u[k]];
+                iA[k] = Real(1) / dA[k];
+                z[k] = r[k] / dA[k];
+                counts[k] = a.inv_src[a.inv_ptr[u[k]]] == (i0 + el) * d + ej;
+                for (int s = 0; s < w.n_shared; ++s)
+                    if (w.shared_u[s] == u[k]) sh[k] = s;
+            }
+        } else {
+            op[k] = -1;
+        }
+    }
+    // this thread's column entries of other workgroups: the word of z, its place in sP
+    const int nk = (ncol * GW + PP_T - 1) / PP_T;                       // at most PP_K
+    int cw[PP_K];
+    Real zc[PP_K];
+#pragma unroll
+    for (int k = 0; k < PP_K; ++k) {
+        const int q = tid + k * PP_T, c = q / GW, cj = q % GW;
+        cw[k] = -1;
+        zc[k] = Real(0);
+        if (c < ncol) {
+            const int img = sCol[c];
+            if ((img < i0 || img >= i1) && cj < d) cw[k] = img * W * GW + cj;
+            sP[q] = Real(0);
+        }
+    }
+    // ---- this lane group's row: blocks part, part + gpr, ... of it, the first NBR in registers (lane = row of
+    // the block), the others in LDS from slot ls on, column-major (a column's lanes read contiguously)
+    const int g = tid / GW, j = tid % GW, row = g / gpr, part = g - row * gpr;
+    int ls0 = 0, ls1 = 0;                                               // this row's LDS slots
+    Real B[NBR + 1][DM];
+    int bx[NBR + 1];                                                        // the column slots of the register blocks
+    {
+        int at = 0;
+        for (int q = 0; q < i1 - i0; ++q) {                             // rows in order: at most 32
+            const int b0 = a.row_ptr[i0 + q] - e0, len = a.row_ptr[i0 + q + 1] - e0 - b0;
+            const int more = max(0, len - NBR * gpr);
+            for (int t = tid; t < more; t += PP_T) sCidx[at + t] = map[col_of(b0 + NBR * gpr + t)] * GW;
+            if (q == row) { ls0 = at; ls1 = at + more; }
+            at += more;                                                 // at most max_blk (ba_pcg_resident_plan)
+        }
+    }
+    const int rb0 = row < i1 - i0 ? a.row_ptr[i0 + row] - e0 : 0, rb1 = row < i1 - i0 ? a.row_ptr[i0 + row + 1] - e0 : 0;
+#pragma unroll
+    for (int k = 0; k < NBR; ++k) {
+        const int b = rb0 + part + k * gpr;
+        const bool live = b < rb1;
+        bx[k] = live ? map[col_of(b)] * GW : 0;
+        const int ent = live ? a.row_ent[e0 + b] : 0;
+        const Real* S = av.S_pairs + (int64_t)(ent >> 1) * dd;
+#pragma unroll
+        for (int c = 0; c < DM; ++c)
+            B[k][c] = live && j < d && c < d ? ((ent & 1) ? S[c * d + j] : S[j * d + c]) : Real(0);
+    }
+    int nbr = 0;                                                        // register blocks of the longest row
+    for (int q = 0; q < i1 - i0; ++q) nbr = max(nbr, (a.row_ptr[i0 + q + 1] - a.row_ptr[i0 + q] + gpr - 1) / gpr);
+    __syncthreads();                                                    // the map is done with
+    {
+        int at = 0;
+        for (int q = 0; q < i1 - i0; ++q) {
+            const int b0 = a.row_ptr[i0 + q] - e0 + NBR * gpr, more = max(0, a.row_ptr[i0 + q + 1] - e0 - b0);
+            for (int t = wave; t < more; t += NW) {                     // one wave per block
+                const int ent = a.row_ent[e0 + b0 + t];
+                const Real* S = av.S_pairs + (int64_t)(ent >> 1) * dd;
+                for (int e = lane; e < dd; e += 64) {
+                    const int c = e / d, rr = e - c * d;
+                    sS[(at + t) * dd + e] = (ent & 1) ? S[c * d + rr] : S[rr * d + c];
+                }
+            }
+            at += more;
+        }
+    }
+    // unknowns without an entry stay 0
+    for (int64_t v = (int64_t)wg * PP_T + tid; v < a.n_u; v += (int64_t)nwg * PP_T)
+        if (a.inv_ptr[v] == a.inv_ptr[v + 1]) av.x[v] = Real(0);
+
+    // Exchange A number ep (first wave): z of the own entries, the workgroup's partials of r.r and r.z.  A
+    // single workgroup leaves the partials in LDS instead.
+    auto publish_a = [&](uint32_t ep) {
+        Real v[2] = {Real(0), Real(0)};
+#pragma unroll
+        for (int k = 0; k < PP_E; ++k) {
+            if (op[k] >= 0 && nwg > 1) {                                // 0 where the entry is no unknown
+#pragma unroll
+                for (int h = 0; h < W; ++h) ll_put(xz + ow[k] + h * GW, L::part(z[k], h), ep);
+            }
+            if (counts[k]) { v[0] += r[k] * r[k]; v[1] += r[k] * z[k]; }
+        }
+        wave_sums(v);
+        if (nwg > 1) xA.put(v, ep, lane);
+        else if (lane == 0) { sA[0] = v[0]; sA[1] = v[1]; }
+    };
+    if (wave == 0) publish_a(1);
+
+    Real bnorm = Real(1), best = INFINITY, rz_old = Real(1), inv_old = Real(1);
+    int bestk = 0, conv_at = 0, n = 0;
+    bool failed = false;
+    for (;; ++n) {
+        const uint32_t ep = (uint32_t)n + 1;
+        // ---- A: the sums of the partials (second wave) and z at the column images (all)
+        if (nwg > 1) {
+            bool good = true;
+            if (wave == 1) {
+                Real v[2] = {Real(0), Real(0)};
+                good = xA.relay(w.limit, ep, lane) && xA.get(w.limit, ep, lane, v);
+                wave_sums(v);
+                if (lane == 0) { sA[0] = v[0]; sA[1] = v[1]; }
+            }
+            good = pp_wait(w.limit, [&]() {
+                uint64_t raw[PP_K][W];
+                bool all = true;
+#pragma unroll
+                for (int k = 0; k < PP_K; ++k)
+                    if (k < nk && cw[k] >= 0)
+#pragma unroll
+                        for (int h = 0; h < W; ++h) raw[k][h] = ll_get(xz + cw[k] + h * GW);
+#pragma unroll
+                for (int k = 0; k < PP_K; ++k)
+                    if (k < nk && cw[k] >= 0) {
+#pragma unroll
+                        for (int h = 0; h < W; ++h) all = all && (uint32_t)(raw[k][h] >> 32) == ep;
+                        zc[k] = L::join(raw[k]);
+                    }
+                return all;
+            }) && good;
+            if (!good) sFailA = 1;
+        } else if (w.limit <= 0) {
+            sFailA = 1;
+        }
+        __syncthreads();
+        const Real rr = sA[0], rz = sA[1];
+        if (sFailA | sFailB) { failed = true; break; }
+        const Real beta = n > 0 ? div_by(rz, rz_old, inv_old) : Real(0);
+#pragma unroll
+        for (int k = 0; k < PP_K; ++k)
+            if (k < nk && cw[k] >= 0) sP[tid + k * PP_T] = pdir(zc[k], sP[tid + k * PP_T], beta);
+        if (wave == 0)
+#pragma unroll
+            for (int k = 0; k < PP_E; ++k)
+                if (op[k] >= 0) { p[k] = pdir(z[k], p[k], beta); sP[op[k]] = p[k]; }
+        __syncthreads();
+        // ---- A p at the own rows: lane group (row, part) takes every gpr-th block of its row
+        Real acc[2] = {Real(0), Real(0)};
+        {
+            Real xk[NBR + 1], xh[NBR + 1];
+#pragma unroll
+            for (int k = 0; k < NBR; ++k)
+                if (k < nbr) {
+                    xk[k] = sP[bx[k] + (tid & 15)];
+                    if constexpr (DM > 16) xh[k] = sP[bx[k] + 16 + (tid & 15)];
+                }
+#pragma unroll
+            for (int k = 0; k < NBR; ++k)
+                if (k < nbr) {
+                    pp_cols<0, DM>([&](int c) { return B[k][c]; }, xk[k], acc);
+                    if constexpr (DM > 16) pp_cols<16, DM>([&](int c) { return B[k][c]; }, xh[k], acc);
+                }
+            for (int b = ls0 + part; b < ls1; b += gpr) {
+                const Real* px = sP + sCidx[b];
+                const Real* Bl = sS + b * dd + (j < d ? j : 0);
+                auto col = [&](int c) { return Bl[min(c, d - 1) * d]; };   // past d, x is 0
+                pp_cols<0, DM>(col, px[tid & 15], acc);
+                if constexpr (DM > 16) pp_cols<16, DM>(col, px[16 + (tid & 15)], acc);
+            }
+        }
+        sY[tid] = acc[0] + acc[1];
+        rz_old = rz > Real(1e-32) ? rz : Real(1e-32);                   // the next update's beta divides by it
+        inv_old = Real(1) / rz_old;
+        // the end of update n - 1 (ba_solver.py:1222-1236); at n = 0 the norm of b
+        const Real rnorm = sqrt(rr);
+        bool stop = false;
+        if (n == 0) {
+            bnorm = rnorm > Real(1e-12) ? rnorm : Real(1e-12);          // torch.norm(b).clamp(min=1e-12)
+        } else {
+            if (rnorm < best) {
+                best = rnorm;
+                bestk = n;
+#pragma unroll
+                for (int k = 0; k < PP_E; ++k) xb_[k] = x[k];
+            }
+            const bool conv = rnorm <= Real(a.tol) * bnorm;
+            if (conv) conv_at = n;
+            stop = conv || !isfinite(rz) || n >= a.maxiter;
+        }
+        __syncthreads();
+        if (stop) break;
+        // ---- B: p.Ap = sum_e p_u(e) y_e + sum_u damp_u p_u^2, and the shared unknowns' sums
+        if (wave == 1 && nwg > 1 && !xB.relay(w.limit, ep, lane)) sFailB = 1;
+        if (wave == 0) {
+            Real q[1 + NS], y[PP_E];
+#pragma unroll
+            for (int s = 0; s <= NS; ++s) q[s] = Real(0);
+#pragma unroll
+            for (int k = 0; k < PP_E; ++k) {
+                y[k] = Real(0);
+                if (u[k] >= 0) {
+                    for (int c = 0; c < gpr; c += 8) {                  // 8 at a time in flight, no branches
+                        Real t[8];
+#pragma unroll
+                        for (int h = 0; h < 8; ++h) t[h] = sY[oy[k] + min(c + h, gpr - 1) * GW];
+#pragma unroll
+                        for (int h = 0; h < 8; ++h) y[k] += c + h < gpr ? t[h] : Real(0);
+                    }
+                    q[0] += p[k] * y[k] + (counts[k] ? dmp[k] * p[k] * p[k] : Real(0));
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) q[1 + s] += sh[k] == s ? y[k] : Real(0);
+                }
+            }
+            wave_sums(q);
+            if (nwg > 1) {
+                xB.put(q, ep, lane);
+                if (!xB.get(w.limit, ep, lane, q)) sFailB = 1;          // read after the next barrier
+                wave_sums(q);
+            }
+            const Real alpha = rz / (q[0] > Real(1e-32) ? q[0] : Real(1e-32));
+#pragma unroll
+            for (int k = 0; k < PP_E; ++k)
+                if (u[k] >= 0) {
+                    Real ap = y[k];
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) ap = sh[k] == s ? q[1 + s] : ap;
+                    ap += dmp[k] * p[k];
+                    x[k] += alpha * p[k];
+                    r[k] -= alpha * ap;
+                    z[k] = div_by(r[k], dA[k], iA[k]);
+                }
+            publish_a(ep + 1);
+        }
+        __syncthreads();         // nobody polls (and so crowds the memory path) before this workgroup has published
+    }
+    if (failed) {
+        if (tid == 0) a.istate[6] = 1;
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < PP_E; ++k)
+        if (u[k] >= 0 && counts[k]) av.x[u[k]] = conv_at ? x[k] : xb_[k];
+    if (wg == 0 && tid == 0) {
+        // the done flags as the launch sequence leaves them: both set after a stop before the cap
+        const int last = (n + 1) & 1;
+        a.istate[last] = 1;
+        a.istate[1 - last] = n < a.maxiter;
+        a.istate[IS_K] = n; a.istate[IS_CONV] = conv_at != 0; a.istate[IS_BESTK] = bestk;
+        a.istate[IS_USEBEST] = conv_at == 0;
+    }
+}
+
 // the flag "stopped before update n" (read once the launches before it have run) to memory the host reads
 // (pinned host memory: a system-scope store)
 __global__ void k_pcg_stopped(const int32_t* __restrict__ flag, int32_t* out) {
@@ -827,6 +1411,107 @@ extern "C" int ba_pcg_solve_pairs_range(const ba_pcg_args* args, const ba_pcg_pa
         BA_REQUIRE(false, "null pairs");
     }
     return pcg_range(args, pairs, it0, it1, finish, stopped_out, stream);
+}
+
+// Images per workgroup of the resident solve (0: it does not apply): of those whose rows fit, the one with the
+// least estimated time of an iteration.  In cycles, measured at 8 to 1024 images: the two exchanges take about
+// 5200 + 50 per workgroup up to 2 PP_G of them, and with relays 9500 + 45 per workgroup; a round of blocks takes 300
+// from registers and 1000 from LDS (the register rounds of the other lane groups hide under it, so the longest row
+// counts); entries beyond the first 64 another 500.
+extern "C" int32_t ba_pcg_resident_plan(const int32_t* row_ptr, int32_t n_imgs, int32_t d, int32_t real32,
+                                        int32_t n_shared, int32_t n_cu, int32_t* max_blk, int32_t* max_col) {
+    if (row_ptr == nullptr || max_blk == nullptr || max_col == nullptr || n_imgs < 1 || n_imgs > 65535 || d < 1 ||
+        d > 32 || n_shared < 0 || n_shared > PP_NS || n_cu < 1)
+        return 0;
+    const int gw = d <= 16 ? 16 : 32, nbr = pp_regs_of(pp_width(d), real32 != 0);
+    const size_t R = real32 ? 4 : 8;
+    int longest = 0, best = 0, best_cost = 0;
+    for (int i = 0; i < n_imgs; ++i) longest = std::max(longest, row_ptr[i + 1] - row_ptr[i]);
+    for (int m = std::min({n_imgs, PP_T / gw, 64 * PP_E / d}); m >= 1; --m) {
+        const int nwg = (n_imgs + m - 1) / m, gpr = PP_T / gw / m;
+        if (nwg > n_cu || nwg > PP_WG) break;
+        int blk = 1, all = 1;
+        for (int i = 0; i < n_imgs; i += m) {
+            int more = 0;
+            const int e = std::min(i + m, n_imgs);
+            for (int q = i; q < e; ++q) more += std::max(0, row_ptr[q + 1] - row_ptr[q] - nbr * gpr);
+            blk = std::max(blk, more);
+            all = std::max(all, row_ptr[e] - row_ptr[i]);
+        }
+        const int col = std::min(all + m, n_imgs);
+        if (col * gw > PP_K * PP_T) continue;
+        if (pp_lds(d, gw, R, n_imgs, blk, col).total > PP_LDS) continue;
+        const int rounds = (longest + gpr - 1) / gpr;
+        const int cost = (nwg == 1 ? 0 : nwg <= 2 * PP_G ? 5200 + 50 * nwg : 9500 + 45 * nwg) +
+                         300 * std::min(rounds, nbr) + 1000 * std::max(0, rounds - nbr) + (m * d > 64 ? 500 : 0);
+        if (best == 0 || cost < best_cost) {
+            best = m;
+            best_cost = cost;
+            *max_blk = blk;
+            *max_col = col;
+        }
+    }
+    return best;
+}
+
+extern "C" int64_t ba_pcg_resident_words(int32_t n_imgs, int32_t d, int32_t real32, int32_t m) {
+    if (n_imgs < 1 || d < 1 || d > 32 || m < 1) return -1;
+    const int64_t gw = d <= 16 ? 16 : 32, nwg = (n_imgs + m - 1) / m;
+    if (nwg > PP_WG) return -1;
+    if (real32) return n_imgs * gw + PpSums<2, float>::words_of((int)nwg) + PpSums<1 + PP_NS, float>::words_of((int)nwg);
+    return 2 * n_imgs * gw + PpSums<2, double>::words_of((int)nwg) + PpSums<1 + PP_NS, double>::words_of((int)nwg);
+}
+
+template <int GW, int DM, int NS, typename Real>
+static int resident_launch(ba_pcg_args a, ba_pcg_resident w, hipStream_t st) {
+    const unsigned nb = nb_of(a.n_u);
+    const unsigned nbw = (unsigned)((a.n_u + PCG_T / 64 - 1) / (PCG_T / 64));
+    const int64_t nw = ba_pcg_resident_words(a.n_imgs, a.d, a.real32, w.m);
+    const void* k = (const void*)k_pcg_resident<GW, DM, NS, Real>;
+    const size_t lds = pp_lds(a.d, GW, sizeof(Real), a.n_imgs, w.max_blk, w.max_col).total;
+    BA_REQUIRE(lds <= PP_LDS, "the image rows do not fit the LDS");
+    BA_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_pp_clear, dim3(nb_of(nw)), dim3(PCG_T), 0, st, w.words, nw, a.istate);
+    hipLaunchKernelGGL(k_unk_setup<Real>, dim3(nbw), dim3(PCG_T), 0, st, a);
+    hipLaunchKernelGGL(k_leaf_max<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
+    hipLaunchKernelGGL(k_leaf_damp<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
+    BA_LAUNCHED();
+    void* args[] = {&a, &w};
+    BA_HIP(hipLaunchCooperativeKernel(k, dim3((unsigned)((a.n_imgs + w.m - 1) / w.m)), dim3(PP_T), args, (unsigned)lds, st));
+    return BA_OK;
+}
+
+template <int NS, typename Real>
+static int resident_width(const ba_pcg_args& a, const ba_pcg_resident& w, hipStream_t st) {
+    switch (pp_width(a.d)) {
+        case 9: return resident_launch<16, 9, NS, Real>(a, w, st);
+        case 13: return resident_launch<16, 13, NS, Real>(a, w, st);
+        case 16: return resident_launch<16, 16, NS, Real>(a, w, st);
+        case 20: return resident_launch<32, 20, NS, Real>(a, w, st);
+        case 25: return resident_launch<32, 25, NS, Real>(a, w, st);
+        default: return resident_launch<32, 32, NS, Real>(a, w, st);
+    }
+}
+
+extern "C" int ba_pcg_solve_resident(const ba_pcg_args* args, const ba_pcg_resident* res, void* stream) {
+    clear_error();
+    BA_REQUIRE(args != nullptr && res != nullptr, "null args");
+    const ba_pcg_args& a = *args;
+    const ba_pcg_resident& w = *res;
+    BA_REQUIRE(a.n_u >= 1 && a.n_imgs >= 1 && a.n_imgs <= 65535 && a.d >= 1 && a.d <= 32 && a.maxiter >= 1 &&
+                   a.maxiter < (1 << 30),
+               "bad sizes (1 <= d <= 32, at most 65535 images, 1 <= maxiter < 2^30)");
+    const void* need[] = {a.umap, a.inv_ptr, a.inv_src, a.leaf, a.row_ptr, a.row_ent, a.pair_i1, a.pair_i2, a.S_pairs,
+                          a.e_img, a.dg_img, a.rhs, a.diagA, a.damp, a.x, a.state, a.istate, w.words};
+    for (const void* q : need) BA_REQUIRE(q != nullptr, "null pointer in ba_pcg_args or ba_pcg_resident");
+    const int gw = a.d <= 16 ? 16 : 32;
+    BA_REQUIRE(w.n_shared >= 0 && w.n_shared <= PP_NS && (w.n_shared == 0 || w.shared_u != nullptr), "bad shared unknowns");
+    BA_REQUIRE(w.m >= 1 && w.m <= PP_T / gw && w.m * a.d <= 64 * PP_E && (a.n_imgs + w.m - 1) / w.m <= PP_WG &&
+                   w.max_blk >= 1 && w.max_col >= 1 && w.max_col * gw <= PP_K * PP_T,
+               "bad resident plan");
+    hipStream_t st = (hipStream_t)stream;
+    if (w.n_shared == 0) return a.real32 ? resident_width<0, float>(a, w, st) : resident_width<0, double>(a, w, st);
+    return a.real32 ? resident_width<PP_NS, float>(a, w, st) : resident_width<PP_NS, double>(a, w, st);
 }
 
 extern "C" int ba_pcg_solve(const ba_pcg_args* args, void* stream) {

@@ -743,7 +743,7 @@ extern "C" int64_t ba_abi_sizeof(const char* name) {
     const std::string n(name);
 #define BA_SZ(T) if (n == #T) return (int64_t)sizeof(T)
     BA_SZ(ba_huber); BA_SZ(ba_layout); BA_SZ(ba_lin_args); BA_SZ(ba_pm_args); BA_SZ(ba_pcg_args);
-    BA_SZ(ba_pcg_pairs);
+    BA_SZ(ba_pcg_pairs); BA_SZ(ba_pcg_resident);
     BA_SZ(ba_chol_args); BA_SZ(ba_sample_args); BA_SZ(ba_obs_set); BA_SZ(ba_gather_args); BA_SZ(ba_remove_args);
     BA_SZ(ba_tangent_args);
 #undef BA_SZ

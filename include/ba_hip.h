@@ -335,6 +335,24 @@ typedef struct {
 } ba_pcg_pairs;
 int ba_pcg_solve_pairs_range(const ba_pcg_args* args, const ba_pcg_pairs* pairs, int32_t it0, int32_t it1,
                              int32_t finish, int32_t* stopped_out, void* stream);
+/* The same solve in one cooperative launch, each workgroup holding m image rows in LDS and exchanging partial
+ * sums and z with the others through `words` (for systems whose rows fit and at most 2 unknowns that several
+ * image-level entries share; the unknowns' lists must ascend, as the planners make them).  istate[6] is set,
+ * and x not, when a wait exceeded `limit`: solve with ba_pcg_solve then.  Of the workspace of args it uses rhs,
+ * diagA, damp, x, state and istate only.  Not for capture into a graph. */
+typedef struct {
+    uint64_t* words;                   /* ba_pcg_resident_words(...) words of workspace */
+    const int32_t* shared_u;           /* (n_shared) the unknowns with two or more image-level entries, all of them */
+    int32_t n_shared;                  /* <= 2 */
+    int32_t m, max_blk, max_col;       /* from ba_pcg_resident_plan */
+    int64_t limit;                     /* longest wait in ticks of 10 ns (0: give up at once) */
+} ba_pcg_resident;
+/* Images per workgroup for the row lists row_ptr (n_imgs + 1, host memory) on a device of n_cu compute units,
+ * with the LDS sizes that go with it (max_blk, max_col); 0 when the resident solve does not apply. */
+int32_t ba_pcg_resident_plan(const int32_t* row_ptr, int32_t n_imgs, int32_t d, int32_t real32, int32_t n_shared,
+                             int32_t n_cu, int32_t* max_blk, int32_t* max_col);
+int64_t ba_pcg_resident_words(int32_t n_imgs, int32_t d, int32_t real32, int32_t m);
+int ba_pcg_solve_resident(const ba_pcg_args* args, const ba_pcg_resident* res, void* stream);
 /* The device address of pinned, mapped host memory (hipPointerGetAttributes), or NULL when the device cannot
  * reach it: the stopped_out target of ba_pcg_solve_range (no counterpart in the reference). */
 void* ba_host_mapped_ptr(const void* host_ptr);

@@ -176,3 +176,93 @@ def test_planners_order_the_pairs_by_image(kind):
             row = ent[row_ptr[i]:row_ptr[i + 1]]
             assert (np.diff(row) > 0).all() and (np.diff(row & 1) <= 0).all()
             assert ((np.where(row & 1, i2[row >> 1], i1[row >> 1])) == i).all()
+
+
+def resident_args(sysm, pa, limit=200_000_000, n_cu=256, m=None):
+    """ba_pcg_resident for a block_system, on m images per workgroup (None: the plan's choice); (res, tensors) or None
+    where the resident solve does not apply."""
+    from blast3r_amd._lib import BaPcgResident, lib
+    flat = sysm['umap'].reshape(-1)
+    counts = np.bincount(flat[flat >= 0], minlength=sysm['n'])
+    shared = np.nonzero(counts >= 2)[0]
+    rp = np.cumsum([0] + [len(r) for r in sysm['rows']]).astype(np.int32)
+    blk, col = ctypes.c_int32(0), ctypes.c_int32(0)
+    plan = lambda cu: lib().ba_pcg_resident_plan(rp.ctypes.data_as(ctypes.c_void_p), sysm['m'], sysm['d'], pa.real32,
+                                                 len(shared), cu, ctypes.byref(blk), ctypes.byref(col))
+    got = plan(n_cu)
+    if got < 1:
+        return None
+    if m is not None:
+        got = min(m, got)
+        blk.value = max(int(rp[min(i + got, sysm['m'])] - rp[i]) for i in range(0, sysm['m'], got))
+        col.value = min(blk.value + got, sysm['m'])
+    nw = int(lib().ba_pcg_resident_words(sysm['m'], sysm['d'], pa.real32, got))
+    words = torch.full((nw,), -1, dtype=torch.int64, device=DEV)
+    sh = torch.as_tensor(shared if len(shared) else np.zeros(1), dtype=torch.int32, device=DEV)
+    res = BaPcgResident(words=words.data_ptr(), shared_u=sh.data_ptr(), n_shared=len(shared), m=got, max_blk=blk.value,
+                        max_col=col.value, limit=limit)
+    return res, (words, sh)
+
+
+RESIDENT = [(1, 13, 2, None), (2, 1, 0, 1), (7, 13, 2, None), (7, 13, 2, 3), (40, 13, 2, 1), (61, 10, 2, None), (256, 9, 0, 1),
+            (250, 13, 2, None), (40, 16, 2, None), (33, 17, 2, None), (30, 25, 2, None), (29, 22, 0, None), (20, 32, 0, 1), (300, 5, 0, 2), (256, 13, 2, 1), (250, 9, 2, None)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('real32', [False, True], ids=['fp64', 'fp32'])
+@pytest.mark.parametrize('m,d,shared,per', RESIDENT)
+def test_resident_solve(m, d, shared, per, real32):
+    """ba_pcg_solve_resident against the oracle's loop after 8 updates (tolerance as above) and, to the end of the loop,
+    against ba_pcg_solve: the same outcome.  One and several workgroups, ragged last ones, one image per workgroup
+    (every column from another workgroup), shared unknowns and parameters that are none, twice in a row."""
+    from blast3r_amd._lib import check, lib, stream_ptr
+    eps = 1.2e-7 if real32 else 2.3e-16
+    for drop in (0.0, 0.3):
+        sysm = block_system(m, d, shared, seed=m * 100 + d, density=0.6 if m < 100 else 0.04, drop=drop,
+                            dtype=np.float32 if real32 else np.float64)
+        if sysm['n'] == 0:
+            continue
+        for maxiter, tol in ((8, 0.0), (100, 1e-4)):
+            pa, keep = pcg_args(sysm, maxiter, tol, real32)
+            got = resident_args(sysm, pa, m=per)
+            assert got is not None
+            res, hold = got
+            print(f'resident m={m} d={d} shared={res.n_shared} per={res.m} blk={res.max_blk} col={res.max_col} drop={drop} '
+                  f'n={sysm["n"]} maxiter={maxiter}', flush=True)
+            check(lib().ba_pcg_solve(ctypes.byref(pa), stream_ptr(DEV)))
+            x_rows, ist_rows = keep['x'].clone(), keep['istate'].cpu()
+            keep['x'].fill_(float('nan'))
+            for _ in range(2):
+                check(lib().ba_pcg_solve_resident(ctypes.byref(pa), ctypes.byref(res), stream_ptr(DEV)))
+            torch.cuda.synchronize()
+            ist = keep['istate'].cpu()
+            assert int(ist[6]) == 0
+            x, _, _ = oracle_iterate(sysm, maxiter, tol)
+            if maxiter == 8:
+                assert float((keep['x'].cpu().double() - x).norm() / x.norm()) < 1e4 * eps
+                assert ist[:6].tolist() == ist_rows[:6].tolist()
+            else:                                      # both meet ||r|| <= tol ||b||; the eigenvalues lie around 1
+                assert int(ist[3]) == int(ist_rows[3]) == 1 and abs(int(ist[2]) - int(ist_rows[2])) <= 1
+                assert float((keep['x'].cpu().double() - x).norm() / x.norm()) < 10 * tol
+
+
+@pytest.mark.gpu
+def test_resident_solve_gives_up_and_the_launch_sequence_takes_over(monkeypatch):
+    """A resident loop whose waits are limited to nothing leaves at once, says so, and solve_delta returns the launch
+    sequence's step; with the usual limit it returns the same step to rounding."""
+    from blast3r_amd import ba_solver, engine
+    from blast3r_amd.synthetic import make_problem
+    p = make_problem(0, n_frames=12, n_tracks=600)
+    kw = dict(dtype=torch.float64, weight_z=1e-2, huber_delta=2.0)
+    steps = {}
+    for limit in (0, ba_solver.RESIDENT_LIMIT):
+        monkeypatch.setattr(ba_solver, 'RESIDENT_LIMIT', limit)
+        g = p.to(DEV)                                  # other tensors: another plan
+        for _ in range(2):
+            info = {}
+            engine._lm_step(**g.lm_inputs(), **kw, info=info)
+            assert info['solver'].last['pcg_resident'] == (limit > 0)
+            assert info['pcg_istate'].cpu()[2] > 0 and info['pcg_istate'].cpu()[6] == 0
+        steps[limit] = info['delta']
+    a, b = steps.values()
+    assert torch.isfinite(a).all() and float((a - b).norm() / b.norm()) < 1e-4
