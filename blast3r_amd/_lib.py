@@ -95,7 +95,7 @@ class BaPmArgs(ctypes.Structure):
                 ('r_in', c_p), ('w_in', c_p), ('r_s0', c_i64), ('r_s1', c_i64), ('w_s0', c_i64), ('w_s1', c_i64),
                 ('pobs', c_p), ('wobs', c_p), ('jslots', c_p), ('vslots', c_p), ('yrun', c_p), ('Hpp', c_p), ('gp', c_p), ('tmax', c_p), ('lam_p', c_p), ('pfac', c_p), ('V', c_p),
                 ('S_pairs', c_p), ('e_img', c_p), ('dg_img', c_p), ('dc_img', c_p), ('dX', c_p), ('dX64', c_p),
-                ('real32', c_int)]
+                ('real32', c_int), ('n_terms', c_i64)]
 
 
 class BaCholArgs(ctypes.Structure):

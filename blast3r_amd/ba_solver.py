@@ -426,7 +426,7 @@ class GaussNewtonSolver:
                      'trk_obs_ptr', 'trk_obs', 'obs_img', 'pair_i1', 'pair_i2', 'diag_pair', 'term_ptr', 'term',
                      'pair_sched'):
             setattr(a, name, ptr(pd[name]))
-        a.n_obs, a.n_runs, a.n_pairs = n_obs, sc['n_runs'], sc['n_pairs']
+        a.n_obs, a.n_runs, a.n_pairs, a.n_terms = n_obs, sc['n_runs'], sc['n_pairs'], sc['n_terms']
         pix = J.pix2d if J.pix2d is not None else J.pix2d_std
         a.pids, a.pix2d, a.pix2d_std, a.pix2d_dep = ptr(J.pids), ptr(pix), ptr(J.pix2d_std), ptr(J.pix2d_dep)
         a.K, a.P_rig2cam, a.P_rig2cam_stride = ptr(J.K), ptr(J.P_rig2cam), J.P_rig2cam.stride(0)

@@ -1696,13 +1696,17 @@ __device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t nb) {
 // once and handed to the row lanes by shuffles, the rows of the next 8 terms are requested before
 // the MFMAs of the current 8.  The pairs are taken in the plan's schedule (pairs whose
 // terms come from the same neighbourhood of images run together and find each other's V rows in the L2)
-template <int DP, typename Real>
+// A term costs two V records from the L2 (2 x 3 DP elements) and the loads of one batch in flight per wave bound the
+// chain of a pair, so long pairs are shared out.  SPLIT: one pair per workgroup, its terms in PM_T / 64 consecutive
+// parts, one per wave, the parts' sums added in order; otherwise one pair per wave.
+template <int DP, bool SPLIT, typename Real>
 __global__ void __launch_bounds__(PM_T) k_pm_pairs(PmArgs a) {
     typedef PmMfma<Real> M;
-    constexpr int NT = DP / 16;
+    constexpr int NT = DP / 16, NW = PM_T / 64;
+    __shared__ typename M::V4 part[SPLIT ? NW - 1 : 1][SPLIT ? NT * NT : 1][SPLIT ? 64 : 1];
     const Real* const Vg = (const Real*)a.V;
-    const int lane = threadIdx.x & 63;
-    const int64_t q = xcd_block(blockIdx.x, gridDim.x) * (PM_T / 64) + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t q = xcd_block(blockIdx.x, gridDim.x) * (SPLIT ? 1 : NW) + (SPLIT ? 0 : wave);
     if (q >= a.n_pairs) return;
     const int64_t p = a.pair_sched != nullptr ? a.pair_sched[q] : q;     // the plan's processing order
     const int i1 = a.pair_i1[p], i2 = a.pair_i2[p];
@@ -1714,14 +1718,19 @@ __global__ void __launch_bounds__(PM_T) k_pm_pairs(PmArgs a) {
     for (int x = 0; x < NT; ++x)
 #pragma unroll
         for (int y = 0; y < NT; ++y) acc[x][y] = (typename M::V4){Real(0), Real(0), Real(0), Real(0)};
-    const int q0 = a.term_ptr[p], q1 = a.term_ptr[p + 1];
+    int q0 = a.term_ptr[p], q1 = a.term_ptr[p + 1];
+    if constexpr (SPLIT) {
+        const int len = ((q1 - q0 + 8 * NW - 1) / (8 * NW)) * 8;             // whole batches; empty past the end
+        q0 = min(q0 + wave * len, q1);
+        q1 = min(q0 + len, q1);
+    }
     const int n = q1 - q0, nbat = (n + 7) >> 3;
     // The loop body has no branches (indices clamped, out-of-range rows zeroed by a factor), so the
     // accumulators stay in the MFMA registers across iterations.
     // term indices of window w (64 terms) in lane order, -1 past the end
     auto window = [&](int w, int& ra, int& rb) {
         const int q = q0 + 64 * w + lane;
-        const int qc = min(q, q1 - 1);
+        const int qc = max(min(q, q1 - 1), 0);
         ra = a.term[2 * (int64_t)qc];
         rb = a.term[2 * (int64_t)qc + 1];
         if (q >= q1) { ra = -1; rb = -1; }
@@ -1766,6 +1775,17 @@ __global__ void __launch_bounds__(PM_T) k_pm_pairs(PmArgs a) {
         window((nb >> 3) + 1, ra_f, rb_f);
         ra_c = wrap ? ra_n : ra_c; rb_c = wrap ? rb_n : rb_c;
         ra_n = wrap ? ra_f : ra_n; rb_n = wrap ? rb_f : rb_n;
+    }
+    if constexpr (SPLIT) {
+        if (wave > 0)
+#pragma unroll
+            for (int t = 0; t < NT * NT; ++t) part[wave - 1][t][lane] = acc[t / NT][t % NT];
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < NW - 1; ++w)
+#pragma unroll
+            for (int t = 0; t < NT * NT; ++t) acc[t / NT][t % NT] += part[w][t][lane];
     }
     Real* S = (Real*)a.S_pairs + p * d * d;
 #pragma unroll
@@ -1867,9 +1887,18 @@ static void pm_stage(const ba_pm_args& a, int stage, hipStream_t st) {
     const bool wide = a.lay.d > 15;
     if (stage == 1) {
         if (a.n_pairs > 0) {
-            const unsigned g = (unsigned)((a.n_pairs + PM_T / 64 - 1) / (PM_T / 64));
-            if (wide) hipLaunchKernelGGL((k_pm_pairs<32, Real>), dim3(g), dim3(PM_T), 0, st, a);
-            else      hipLaunchKernelGGL((k_pm_pairs<16, Real>), dim3(g), dim3(PM_T), 0, st, a);
+            // A workgroup per pair where the pairs' chains of terms are long, or too few to hold the chip; four
+            // waves started, drained and joined for short ones cost more than they save.  Measured, a wave / a
+            // workgroup per pair, us: d = 11 fp64 at 56 terms a pair 47 / 46, 87: 203 / 226, 149: 184 / 170, 400:
+            // 124 / 107, 700: 530 / 464; fp32 at 84: 158 / 219, 112: 53 / 53, 520: 62 / 26; d = 23 fp64 at 34: 61 /
+            // 59, 67: 104 / 88, 830: 1239 / 916; fp32 at 34: 40 / 50, 67: 68 / 63; 820 pairs of 40: 10.3 / 8.4
+            // (fp32 8.4 / 8.4), 36 of 118: 14.0 / 6.2
+            const bool split = a.n_terms >= (a.n_pairs <= 1024 ? 32 : wide ? 64 : 128) * a.n_pairs;
+            const unsigned g = (unsigned)(split ? a.n_pairs : (a.n_pairs + PM_T / 64 - 1) / (PM_T / 64));
+            if (wide && split)  hipLaunchKernelGGL((k_pm_pairs<32, true, Real>), dim3(g), dim3(PM_T), 0, st, a);
+            else if (wide)      hipLaunchKernelGGL((k_pm_pairs<32, false, Real>), dim3(g), dim3(PM_T), 0, st, a);
+            else if (split)     hipLaunchKernelGGL((k_pm_pairs<16, true, Real>), dim3(g), dim3(PM_T), 0, st, a);
+            else                hipLaunchKernelGGL((k_pm_pairs<16, false, Real>), dim3(g), dim3(PM_T), 0, st, a);
         }
         return;
     }

@@ -250,6 +250,8 @@ typedef struct {
      * throughout (its dtype=torch.float32 default, ba_solver.py:22, :37, :128): the Jacobian core is
      * evaluated in fp64 and rounded, every product, sum and factor after it is fp32 */
     int32_t real32;
+    int64_t n_terms;                         /* terms of all pairs (term_ptr[n_pairs]): chooses how k_pm_pairs shares
+                                              * them out; 0 = not known */
 } ba_pm_args;
 
 int ba_pm_linearize_schur(const ba_pm_args* args, void* stream);
