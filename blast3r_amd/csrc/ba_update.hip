@@ -97,13 +97,12 @@ __global__ void __launch_bounds__(256) k_apply_update(const float* __restrict__ 
 }
 
 // ------------------------------------------------------------------ objective
-#define OBJ_T 256
-#define OBJ_NBMAX 2048
-
-__global__ void k_obj_init(uint32_t* __restrict__ hist, uint32_t* __restrict__ sel, uint32_t k) {
-    hist[threadIdx.x] = 0;
-    if (threadIdx.x == 0) { sel[0] = 0; sel[1] = 0; sel[2] = k; sel[3] = 0; }
-}
+#define OBJ_T 512
+#define OBJ_NB 512        // most blocks of a pass: two per CU, 8 waves each
+#define OBJ_SMALL 16384   // observations up to which one workgroup does it all
+#define OBJ_SMALL_T 1024
+#define OBJ_COPIES 16     // of the histogram in memory, block b adds to copy b % 16: the values cluster in few bins
+#define OBJ_SUBH 16       // and in LDS (lane & 15; rows 257 words apart, so a bin's copies lie in different banks)
 
 // the selection key of observation i: the bit pattern of ||(r0, r1)|| (non-negative, so the pattern
 // orders as the value).  Every kernel forms it through this one function, so a key stored by
@@ -113,57 +112,29 @@ __device__ __forceinline__ uint32_t obj_key(const float* __restrict__ res, int64
     return __float_as_uint(sqrtf(r0 * r0 + r1 * r1));
 }
 
-__global__ void __launch_bounds__(OBJ_T) k_obj_prep(const float* __restrict__ res, int64_t n, int has_err,
-                                                   uint32_t* __restrict__ ebits, double* __restrict__ part) {
-    __shared__ double sh[OBJ_T];
-    double s = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * OBJ_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * OBJ_T) {
-        if (ebits) ebits[i] = obj_key(res, n, i);
-        if (has_err) s += (double)res[3 * n + i] + (double)res[4 * n + i] + (double)res[5 * n + i];
-    }
-    sh[threadIdx.x] = s;
+// The sum over the block (all threads get it): the waves by an xor tree, then their sums in order.
+template <int T, typename V>
+__device__ __forceinline__ V obj_block_sum(V v, V* sh) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
     __syncthreads();
-    for (int w = OBJ_T / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    V t = sh[0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) t += sh[w];
+    return t;
 }
 
-// histogram of the next 8 bits among values whose higher bits equal the prefix.  The values cluster
-// in few bins (the top byte is the exponent), so each block keeps 8 sub-histograms (lane & 7; rows
-// 257 words apart, so a bin's copies lie in different LDS banks) to spread the atomic increments.
-#define OBJ_SUBH 8
-__global__ void __launch_bounds__(OBJ_T) k_obj_hist(const uint32_t* __restrict__ ebits, const float* __restrict__ res,
-                                                   int64_t n, const uint32_t* __restrict__ sel, int shift,
-                                                   uint32_t* __restrict__ hist) {
-    __shared__ uint32_t h[OBJ_SUBH][257];
-#pragma unroll
-    for (int k = 0; k < OBJ_SUBH; ++k) h[k][threadIdx.x] = 0;
-    __syncthreads();
-    uint32_t prefix = sel[0], pmask = sel[1];
-    uint32_t* mine = h[threadIdx.x & (OBJ_SUBH - 1)];
-    for (int64_t i = (int64_t)blockIdx.x * OBJ_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * OBJ_T) {
-        uint32_t b = ebits ? ebits[i] : obj_key(res, n, i);
-        if ((b & pmask) == prefix) atomicAdd(&mine[(b >> shift) & 0xffu], 1u);
-    }
-    __syncthreads();
-    uint32_t t = 0;
-#pragma unroll
-    for (int k = 0; k < OBJ_SUBH; ++k) t += h[k][threadIdx.x];
-    if (t) atomicAdd(&hist[threadIdx.x], t);
-}
-
-// pick the bin holding the k-th smallest (k in sel[2], 1-based); clear hist for the next pass
-// One wave: lane l holds bins 4l .. 4l + 3; an inclusive scan of the lane sums finds the lane, then
-// the bin, where the running count first reaches k (the same bin and count as a sequential walk;
-// when no bin reaches k: bin 255 with the full count, as that walk leaves them).
-__global__ void __launch_bounds__(64) k_obj_pick(uint32_t* __restrict__ hist, uint32_t* __restrict__ sel, int shift) {
-    const int l = threadIdx.x;
-    const uint32_t k = sel[2];
+// One step of the selection, one wave: the bin of h (256 counters) holding the k-th smallest (1-based) goes into the
+// prefix, the ranks below it leave k.  Lane l holds bins 4l .. 4l + 3; an inclusive scan of the lane sums finds the
+// lane, then the bin, where the running count first reaches k (the same bin and count as a sequential walk; when no
+// bin reaches k: bin 255 with the full count, as that walk leaves them).
+__device__ __forceinline__ void obj_pick(const uint32_t* h256, int shift, uint32_t& prefix, uint32_t& k) {
+    const int l = threadIdx.x & 63;
     uint32_t h[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) h[q] = hist[4 * l + q];
+    for (int q = 0; q < 4; ++q) h[q] = h256[4 * l + q];
     const uint32_t s = h[0] + h[1] + h[2] + h[3];
     uint32_t inc = s;
 #pragma unroll
@@ -188,59 +159,213 @@ __global__ void __launch_bounds__(64) k_obj_pick(uint32_t* __restrict__ hist, ui
         b = 4 * L + q;
         cum = c;
     }
-    if (l == 0) {
-        sel[0] |= (uint32_t)b << shift;
-        sel[1] |= 0xffu << shift;
-        sel[2] = k - cum;
-    }
+    prefix |= (uint32_t)b << shift;
+    k -= cum;
+}
+
+// counters of the selection's four digits and, per digit, the prefix and rank before it
+struct ObjSel {
+    uint32_t hist[4][OBJ_COPIES][256];
+    uint32_t state[5][2];
+};
+
+__global__ void __launch_bounds__(256) k_obj_init(ObjSel* __restrict__ o, uint32_t k) {
+    (&o->hist[0][0][0])[blockIdx.x * 256 + threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) { o->state[0][0] = 0; o->state[0][1] = k; }
+}
+
+__device__ __forceinline__ void obj_hist_clear(uint32_t (&h)[OBJ_SUBH][257], int nt) {
+    for (int t = threadIdx.x; t < OBJ_SUBH * 257; t += nt) (&h[0][0])[t] = 0;
+    __syncthreads();
+}
+__device__ __forceinline__ uint32_t obj_hist_bin(uint32_t (&h)[OBJ_SUBH][257], int bin) {
+    uint32_t t = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) hist[4 * l + q] = 0;
+    for (int k = 0; k < OBJ_SUBH; ++k) t += h[k][bin];
+    return t;
+}
+__device__ __forceinline__ void obj_hist_flush(uint32_t (&h)[OBJ_SUBH][257], ObjSel* o, int digit) {
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        const uint32_t t = obj_hist_bin(h, threadIdx.x);
+        if (t) atomicAdd(&o->hist[digit][blockIdx.x % OBJ_COPIES][threadIdx.x], t);
+    }
+}
+
+// Keys of all observations (4 in flight per thread), the histogram of their top byte, and the block's partial of
+// sum(err).  Keys need no second launch for their first digit: nothing is selected before it.
+__global__ void __launch_bounds__(OBJ_T) k_obj_prep(const float* __restrict__ res, int64_t n, int has_err,
+                                                   uint32_t* __restrict__ ebits, double* __restrict__ part,
+                                                   ObjSel* __restrict__ o) {
+    __shared__ uint32_t h[OBJ_SUBH][257];
+    __shared__ double sh[OBJ_T / 64];
+    obj_hist_clear(h, OBJ_T);
+    uint32_t* mine = h[threadIdx.x & (OBJ_SUBH - 1)];
+    const int64_t step = (int64_t)gridDim.x * OBJ_T;
+    double s = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * OBJ_T + threadIdx.x; i < n; i += 4 * step) {
+        uint32_t key[4];
+        float e[4][3];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = i + u * step < n ? i + u * step : n - 1;
+            key[u] = obj_key(res, n, q);
+            if (has_err) { e[u][0] = res[3 * n + q]; e[u][1] = res[4 * n + q]; e[u][2] = res[5 * n + q]; }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * step < n) {
+                if (ebits) ebits[i + u * step] = key[u];
+                if (has_err) s += (double)e[u][0] + (double)e[u][1] + (double)e[u][2];
+                atomicAdd(&mine[key[u] >> 24], 1u);
+            }
+    }
+    obj_hist_flush(h, o, 0);
+    s = obj_block_sum<OBJ_T>(s, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// the selection after `digits` digits, made by every block for itself (16 KB from the L2, one scan) so that it needs
+// no launch of its own; block 0 writes it down for the next pass
+__device__ __forceinline__ void obj_select(ObjSel* __restrict__ o, int digits, uint32_t (&hs)[256], uint32_t (&st)[2]) {
+    if (threadIdx.x < 256) {
+        uint32_t t = 0;
+#pragma unroll
+        for (int c = 0; c < OBJ_COPIES; ++c) t += o->hist[digits - 1][c][threadIdx.x];
+        hs[threadIdx.x] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        uint32_t prefix = o->state[digits - 1][0], k = o->state[digits - 1][1];
+        obj_pick(hs, 32 - 8 * digits, prefix, k);
+        if (threadIdx.x == 0) {
+            st[0] = prefix;
+            st[1] = k;
+            if (blockIdx.x == 0) { o->state[digits][0] = prefix; o->state[digits][1] = k; }
+        }
+    }
+    __syncthreads();
+}
+
+// histogram of digit `digit` (1 .. 3) among the keys whose higher digits are the selected ones
+__global__ void __launch_bounds__(OBJ_T) k_obj_hist(const uint32_t* __restrict__ ebits, const float* __restrict__ res,
+                                                   int64_t n, int digit, ObjSel* __restrict__ o) {
+    __shared__ uint32_t h[OBJ_SUBH][257], hs[256], st[2];
+    obj_hist_clear(h, OBJ_T);
+    obj_select(o, digit, hs, st);
+    const int shift = 24 - 8 * digit;
+    const uint32_t prefix = st[0] >> (shift + 8);
+    uint32_t* mine = h[threadIdx.x & (OBJ_SUBH - 1)];
+    const int64_t step = (int64_t)gridDim.x * OBJ_T;
+    for (int64_t i = (int64_t)blockIdx.x * OBJ_T + threadIdx.x; i < n; i += 4 * step) {
+        uint32_t key[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = i + u * step < n ? i + u * step : n - 1;
+            key[u] = ebits ? ebits[q] : obj_key(res, n, q);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * step < n && (key[u] >> (shift + 8)) == prefix) atomicAdd(&mine[(key[u] >> shift) & 0xffu], 1u);
+    }
+    obj_hist_flush(h, o, digit);
 }
 
 __global__ void __launch_bounds__(OBJ_T) k_obj_below(const uint32_t* __restrict__ ebits, const float* __restrict__ res,
-                                                    int64_t n, const uint32_t* __restrict__ sel,
-                                                    double* __restrict__ psum, uint32_t* __restrict__ pcnt) {
-    __shared__ double sh[OBJ_T];
-    __shared__ uint32_t sc[OBJ_T];
-    uint32_t T = sel[0];
+                                                    int64_t n, ObjSel* __restrict__ o, double* __restrict__ psum,
+                                                    uint32_t* __restrict__ pcnt) {
+    __shared__ uint32_t hs[256], st[2], sc[OBJ_T / 64];
+    __shared__ double sh[OBJ_T / 64];
+    obj_select(o, 4, hs, st);
+    const uint32_t T = st[0];
+    const int64_t step = (int64_t)gridDim.x * OBJ_T;
     double s = 0.0;
     uint32_t c = 0;
-    for (int64_t i = (int64_t)blockIdx.x * OBJ_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * OBJ_T) {
-        uint32_t b = ebits ? ebits[i] : obj_key(res, n, i);
-        if (b < T) { s += (double)__uint_as_float(b); c += 1; }
+    for (int64_t i = (int64_t)blockIdx.x * OBJ_T + threadIdx.x; i < n; i += 4 * step) {
+        uint32_t key[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = i + u * step < n ? i + u * step : n - 1;
+            key[u] = ebits ? ebits[q] : obj_key(res, n, q);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * step < n && key[u] < T) { s += (double)__uint_as_float(key[u]); c += 1; }
     }
-    sh[threadIdx.x] = s; sc[threadIdx.x] = c;
-    __syncthreads();
-    for (int w = OBJ_T / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) { sh[threadIdx.x] += sh[threadIdx.x + w]; sc[threadIdx.x] += sc[threadIdx.x + w]; }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) { psum[blockIdx.x] = sh[0]; pcnt[blockIdx.x] = sc[0]; }
+    s = obj_block_sum<OBJ_T>(s, sh);
+    c = obj_block_sum<OBJ_T>(c, sc);
+    if (threadIdx.x == 0) { psum[blockIdx.x] = s; pcnt[blockIdx.x] = c; }
 }
 
+// out from the sums: lsum = sum(err), s and c = the sum and number of the keys below the threshold key
+__device__ __forceinline__ void obj_out(double lsum, double s, uint64_t c, uint32_t key, int64_t n, int64_t n80,
+                                        int has_err, float* out) {
+    const double tot = s + (double)(n80 - (int64_t)c) * (double)__uint_as_float(key);
+    out[0] = has_err ? (float)(lsum / (3.0 * (double)n)) : NAN;
+    out[1] = n80 > 0 ? (float)(tot / (double)n80) : NAN;
+}
+
+// the blocks' partials: one per thread
 __global__ void __launch_bounds__(OBJ_T) k_obj_final(const double* __restrict__ lpart, const double* __restrict__ psum,
-                                                    const uint32_t* __restrict__ pcnt, int nb, int64_t n,
-                                                    int64_t n80, const uint32_t* __restrict__ sel, int has_err,
-                                                    float* __restrict__ out) {
-    __shared__ double sh[OBJ_T], sl[OBJ_T];
-    __shared__ uint64_t sc[OBJ_T];
-    double s = 0.0, l = 0.0;
-    uint64_t c = 0;
-    for (int b = threadIdx.x; b < nb; b += OBJ_T) { s += psum[b]; l += lpart[b]; c += pcnt[b]; }
-    sh[threadIdx.x] = s; sl[threadIdx.x] = l; sc[threadIdx.x] = c;
-    __syncthreads();
-    for (int w = OBJ_T / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            sh[threadIdx.x] += sh[threadIdx.x + w]; sl[threadIdx.x] += sl[threadIdx.x + w]; sc[threadIdx.x] += sc[threadIdx.x + w];
+                                                    const uint32_t* __restrict__ pcnt, int nb, int64_t n, int64_t n80,
+                                                    const ObjSel* __restrict__ o, int has_err, float* __restrict__ out) {
+    static_assert(OBJ_NB <= OBJ_T, "one partial per thread");
+    __shared__ double sh[OBJ_T / 64];
+    __shared__ uint64_t sc[OBJ_T / 64];
+    const int b = threadIdx.x;
+    const double s = obj_block_sum<OBJ_T>(b < nb ? psum[b] : 0.0, sh), l = obj_block_sum<OBJ_T>(b < nb ? lpart[b] : 0.0, sh);
+    const uint64_t c = obj_block_sum<OBJ_T>(b < nb ? (uint64_t)pcnt[b] : (uint64_t)0, sc);
+    if (b == 0) obj_out(l, s, c, o->state[4][0], n, n80, has_err, out);
+}
+
+// The whole objective of at most OBJ_SMALL observations in one workgroup: the keys stay in registers.
+__global__ void __launch_bounds__(OBJ_SMALL_T) k_obj_small(const float* __restrict__ res, int n, int has_err, int64_t n80,
+                                                          float* __restrict__ out) {
+    constexpr int PER = OBJ_SMALL / OBJ_SMALL_T;
+    __shared__ uint32_t h[OBJ_SUBH][257], hs[256], st[2];
+    __shared__ double sh[OBJ_SMALL_T / 64];
+    __shared__ uint32_t sc[OBJ_SMALL_T / 64];
+    uint32_t key[PER];
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = threadIdx.x + u * OBJ_SMALL_T;
+        key[u] = 0;
+        if (i < n) {
+            key[u] = obj_key(res, n, i);
+            if (has_err) s += (double)res[3 * (int64_t)n + i] + (double)res[4 * (int64_t)n + i] + (double)res[5 * (int64_t)n + i];
+        }
+    }
+    const double lsum = obj_block_sum<OBJ_SMALL_T>(s, sh);
+    uint32_t prefix = 0, k = (uint32_t)(n80 > 0 ? n80 : 1);
+    for (int digit = 0; digit < 4; ++digit) {
+        const int shift = 24 - 8 * digit;
+        const uint32_t high = digit > 0 ? 0xffffffffu << (shift + 8) : 0u;
+        obj_hist_clear(h, OBJ_SMALL_T);
+        uint32_t* mine = h[threadIdx.x & (OBJ_SUBH - 1)];
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if ((int)threadIdx.x + u * OBJ_SMALL_T < n && (key[u] & high) == prefix)
+                atomicAdd(&mine[(key[u] >> shift) & 0xffu], 1u);
+        __syncthreads();
+        if (threadIdx.x < 256) hs[threadIdx.x] = obj_hist_bin(h, threadIdx.x);
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            obj_pick(hs, shift, prefix, k);
+            if (threadIdx.x == 0) { st[0] = prefix; st[1] = k; }
         }
         __syncthreads();
+        prefix = st[0];
+        k = st[1];
     }
-    if (threadIdx.x == 0) {
-        float T = __uint_as_float(sel[0]);
-        double tot = sh[0] + (double)(n80 - (int64_t)sc[0]) * (double)T;
-        out[0] = has_err ? (float)(sl[0] / (3.0 * (double)n)) : NAN;
-        out[1] = n80 > 0 ? (float)(tot / (double)n80) : NAN;
-    }
+    s = 0.0;
+    uint32_t c = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u)
+        if ((int)threadIdx.x + u * OBJ_SMALL_T < n && key[u] < prefix) { s += (double)__uint_as_float(key[u]); c += 1; }
+    s = obj_block_sum<OBJ_SMALL_T>(s, sh);
+    c = obj_block_sum<OBJ_SMALL_T>(c, sc);
+    if (threadIdx.x == 0) obj_out(lsum, s, c, prefix, n, n80, has_err, out);
 }
 
 // ------------------------------------------------------------------ input checks
@@ -357,53 +482,49 @@ extern "C" int ba_apply_update(const float* K, const float* P_w2rig, const float
 }
 
 extern "C" int64_t ba_objective_workspace_bytes(int64_t n_obs) {
-    int64_t nb = (n_obs + OBJ_T - 1) / OBJ_T;
-    if (nb < 1) nb = 1;
-    return 4 * n_obs + 8 * nb * 2 + 4 * nb + 4 * 256 + 4 * 4 + 64;
+    return 4 * n_obs + OBJ_NB * (8 + 8 + 4) + (int64_t)sizeof(ObjSel) + 64;
 }
 
 namespace ba {
 
 // The launch sequence of ba_objective.  ebits (4 bytes per observation) keeps each observation's
 // key between the passes; when it is null the passes recompute the key from res instead.  lpart,
-// psum (fp64) and pcnt hold one partial per block of the grid-stride passes (at most OBJ_NBMAX),
-// hist 256 counters, sel 4 words; k_obj_init clears hist and sel, every partial is written before
-// it is read.
+// psum (fp64) and pcnt hold one partial per block of the grid-stride passes (at most OBJ_NB); k_obj_init
+// clears the counters, every partial is written before it is read.
+//
+// All of it is latency: a few MB that the residual pass has just left in the caches, about 3 us a launch.  One
+// workgroup up to OBJ_SMALL observations (16384: 15.7 us, the launches 22.9), 7 launches past that.  Measured
+// against 12 launches (the digits' picks on their own, up to 1024 blocks adding to one histogram of few used bins, the
+// top byte apart from the keys), us: 300 observations 33.7 -> 8.8, 16384: 40.7 -> 15.7, 65000: 38.6 -> 24.2,
+// 262144: 57.7 -> 24.8, 1 M: 86.3 -> 26.1, 2.6 M: 102 -> 36.9.
 static int objective_launch(const float* res, int64_t n_obs, int32_t has_err, uint32_t* ebits, double* lpart,
-                            double* psum, uint32_t* pcnt, uint32_t* hist, uint32_t* sel, float* out, hipStream_t st) {
-    int64_t nb = (n_obs + OBJ_T - 1) / OBJ_T;
-    if (nb < 1) nb = 1;
-    int64_t n80 = n_obs * 80 / 100;
+                            double* psum, uint32_t* pcnt, ObjSel* o, float* out, hipStream_t st) {
+    const int64_t n80 = n_obs * 80 / 100;
     BA_REQUIRE(n80 <= (int64_t)UINT32_MAX, "ba_objective: the 80% rank of n_obs must fit 32 bits "
                                           "(n_obs <= 5368709119)");
-    // the per-block partials of prep and below: at most OBJ_NBMAX blocks (grid-stride loops), so the
-    // one-block final sum stays short
-    const int64_t nbp = nb < OBJ_NBMAX ? nb : OBJ_NBMAX;
-    hipLaunchKernelGGL(k_obj_init, dim3(1), dim3(256), 0, st, hist, sel, (uint32_t)(n80 > 0 ? n80 : 1));
-    if (n_obs > 0) {
-        hipLaunchKernelGGL(k_obj_prep, dim3((unsigned)nbp), dim3(OBJ_T), 0, st, res, n_obs, has_err, ebits, lpart);
-        unsigned hb = (unsigned)(nb < 1024 ? nb : 1024);
-        for (int pass = 0; pass < 4; ++pass) {
-            int shift = 24 - 8 * pass;
-            hipLaunchKernelGGL(k_obj_hist, dim3(hb), dim3(OBJ_T), 0, st, ebits, res, n_obs, sel, shift, hist);
-            hipLaunchKernelGGL(k_obj_pick, dim3(1), dim3(64), 0, st, hist, sel, shift);
-        }
-        hipLaunchKernelGGL(k_obj_below, dim3((unsigned)nbp), dim3(OBJ_T), 0, st, ebits, res, n_obs, sel, psum, pcnt);
-    } else {
-        hipLaunchKernelGGL(k_obj_prep, dim3(1), dim3(OBJ_T), 0, st, res, (int64_t)0, has_err, ebits, lpart);
-        hipLaunchKernelGGL(k_obj_below, dim3(1), dim3(OBJ_T), 0, st, ebits, res, (int64_t)0, sel, psum, pcnt);
+    if (n_obs <= OBJ_SMALL) {
+        hipLaunchKernelGGL(k_obj_small, dim3(1), dim3(OBJ_SMALL_T), 0, st, res, (int)n_obs, has_err, n80, out);
+        BA_LAUNCHED();
+        return BA_OK;
     }
-    hipLaunchKernelGGL(k_obj_final, dim3(1), dim3(OBJ_T), 0, st, lpart, psum, pcnt, n_obs > 0 ? (int)nbp : 1, n_obs,
-                       n80, sel, has_err, out);
+    const int64_t nb = (n_obs + OBJ_T - 1) / OBJ_T;
+    const dim3 g((unsigned)(nb < OBJ_NB ? nb : OBJ_NB));
+    hipLaunchKernelGGL(k_obj_init, dim3(4 * OBJ_COPIES), dim3(256), 0, st, o, (uint32_t)n80);
+    hipLaunchKernelGGL(k_obj_prep, g, dim3(OBJ_T), 0, st, res, n_obs, has_err, ebits, lpart, o);
+    for (int digit = 1; digit < 4; ++digit)
+        hipLaunchKernelGGL(k_obj_hist, g, dim3(OBJ_T), 0, st, ebits, res, n_obs, digit, o);
+    hipLaunchKernelGGL(k_obj_below, g, dim3(OBJ_T), 0, st, ebits, res, n_obs, o, psum, pcnt);
+    hipLaunchKernelGGL(k_obj_final, dim3(1), dim3(OBJ_T), 0, st, lpart, psum, pcnt, (int)g.x, n_obs, n80, o, has_err,
+                       out);
     BA_LAUNCHED();
     return BA_OK;
 }
 
 // Scratch of ba_objective_noalloc: the fixed-size part of the objective's workspace (the per-block
-// partials, histogram and selection state; no per-observation keys), one copy per GPU for the life
+// partials, histograms and selection state; no per-observation keys), one copy per GPU for the life
 // of the process.  Host code never uses the symbol itself: each device's address comes from
 // hipGetSymbolAddress, taken once per device with that device current.
-#define OBJ_SCRATCH_BYTES (OBJ_NBMAX * (8 + 8 + 4) + 256 * 4 + 4 * 4)
+#define OBJ_SCRATCH_BYTES (OBJ_NB * (8 + 8 + 4) + sizeof(ObjSel))
 static __device__ __align__(256) unsigned char scratch[(OBJ_SCRATCH_BYTES + 255) / 256 * 256];
 
 #define OBJ_MAX_DEVICES 64
@@ -433,17 +554,13 @@ extern "C" int ba_objective(const float* res, int64_t n_obs, int32_t has_err, vo
                             void* stream) {
     clear_error();
     BA_REQUIRE(n_obs >= 0, "ba_objective: n_obs < 0");
-    int64_t nb = (n_obs + OBJ_T - 1) / OBJ_T;
-    if (nb < 1) nb = 1;
     char* w = (char*)workspace;
     uint32_t* ebits = (uint32_t*)w; w += 4 * n_obs;
     w = (char*)(((uintptr_t)w + 7) & ~(uintptr_t)7);
-    double* lpart = (double*)w; w += 8 * nb;
-    double* psum = (double*)w; w += 8 * nb;
-    uint32_t* pcnt = (uint32_t*)w; w += 4 * nb;
-    uint32_t* hist = (uint32_t*)w; w += 4 * 256;
-    uint32_t* sel = (uint32_t*)w;
-    return objective_launch(res, n_obs, has_err, ebits, lpart, psum, pcnt, hist, sel, out, (hipStream_t)stream);
+    double* lpart = (double*)w; w += 8 * OBJ_NB;
+    double* psum = (double*)w; w += 8 * OBJ_NB;
+    uint32_t* pcnt = (uint32_t*)w; w += 4 * OBJ_NB;
+    return objective_launch(res, n_obs, has_err, ebits, lpart, psum, pcnt, (ObjSel*)w, out, (hipStream_t)stream);
 }
 
 // ba_objective with no workspace argument and no allocation: the passes recompute each key from res
@@ -456,9 +573,8 @@ extern "C" int ba_objective_noalloc(const float* res, int64_t n_obs, int32_t has
     int rc = scratch_of_current_device(&sp);
     if (rc != BA_OK) return rc;
     double* lpart = (double*)sp;
-    double* psum = lpart + OBJ_NBMAX;
-    uint32_t* pcnt = (uint32_t*)(psum + OBJ_NBMAX);
-    uint32_t* hist = pcnt + OBJ_NBMAX;
-    uint32_t* sel = hist + 256;
-    return objective_launch(res, n_obs, has_err, nullptr, lpart, psum, pcnt, hist, sel, out, (hipStream_t)stream);
+    double* psum = lpart + OBJ_NB;
+    uint32_t* pcnt = (uint32_t*)(psum + OBJ_NB);
+    return objective_launch(res, n_obs, has_err, nullptr, lpart, psum, pcnt, (ObjSel*)(pcnt + OBJ_NB), out,
+                            (hipStream_t)stream);
 }
