@@ -55,6 +55,7 @@ _LIN_FIELDS = [
     ('ct_pt', c_p), ('n_ctracks', c_i64), ('core', c_p),
     ('chunk_slots', c_p), ('chunk_ent', c_p), ('chunk_eptr', c_p), ('b_pos_slot', c_p), ('pfac', c_p),
     ('b_order', c_p), ('work_ctr', c_p), ('dc_img', c_p), ('real32', c_int),
+    ('parts', c_int), ('n_slots', c_i64),
 ]
 
 
@@ -192,6 +193,7 @@ _SIGS = {
     'ba_pm_plan_query': (c_int, [c_p, c_p, c_p]),
     'ba_pm_plan_export': (c_int, [c_p, c_int, c_p]),
     'ba_pm_plan_destroy': (None, [c_p]),
+    'ba_schur_parts': (ctypes.c_int32, [c_i64, c_i64, c_i64, ctypes.c_int32]),
     'ba_pm_linearize_schur': (c_int, [ctypes.POINTER(BaPmArgs), c_p]),
     'ba_pm_linearize_stage': (c_int, [ctypes.POINTER(BaPmArgs), c_int, c_p]),
     'ba_pm_backsubstitute': (c_int, [ctypes.POINTER(BaPmArgs), c_p]),

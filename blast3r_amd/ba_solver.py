@@ -327,8 +327,10 @@ class GaussNewtonSolver:
         chunk_max = ws('chunk_max', (sc['n_chunks'] + 1,), R)
         lam_p = ws('lam_p', (1,), R)
         dd = max(d, 1)
-        partials = ws('partials', (max(sc['n_slots'], 1), dd, dd), R)
-        img_partials = ws('img_partials', (max(sc['n_batches'], 1), plan.L, 2, dd), R)
+        n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+        parts = int(lib().ba_schur_parts(sc['n_batches'], sc['n_chunks'], sc['max_chunks_per_batch'], n_cu))
+        partials = ws('partials', (parts, max(sc['n_slots'], 1), dd, dd), R)
+        img_partials = ws('img_partials', (parts, max(sc['n_batches'], 1), plan.L, 2, dd), R)
         # outputs live in the plan's workspace: fixed addresses across LM steps (graph replay)
         S_pairs = ws('S_pairs', (max(sc['n_pairs'], 1), dd, dd), R)
         e_img = ws('e_img', (n_imgs, dd), R)
@@ -370,6 +372,7 @@ class GaussNewtonSolver:
         a.ct_pt, a.n_ctracks, a.core, a.pfac = ptr(ct_pt), n_ct, ptr(core), ptr(pfac)
         a.work_ctr = ptr(work_ctr)
         a.partials, a.img_partials = ptr(partials), ptr(img_partials)
+        a.parts, a.n_slots = parts, sc['n_slots']
         a.n_chunks, a.n_batches, a.n_pairs = sc['n_chunks'], sc['n_batches'], sc['n_pairs']
         a.S_pairs, a.e_img, a.dg_img = ptr(S_pairs), ptr(e_img), ptr(dg_img)
         # residuals / weights: recompute in-kernel when they are this step's own objective output,

@@ -697,11 +697,24 @@ __global__ void __launch_bounds__(BA_WAVES * 64) k_schur(LinArgs a) {
         __syncthreads();
         bq = sNext;
     }
-    if (bq >= a.n_batches) break;
-    const int batch = a.b_order != nullptr ? a.b_order[bq] : bq;             // most expensive first
+    // work item = a part of a batch's chunks, with partials of its own (lin_stage)
+    const int item = __builtin_amdgcn_readfirstlane(bq), parts = max(a.parts, 1);
+    if (item >= a.n_batches * parts) break;
+    const int bo = item / parts, part = item - bo * parts;
+    const int batch = a.b_order != nullptr ? a.b_order[bo] : bo;             // most expensive first
     const int nimg = a.b_nimgs[batch];
     const int s0 = a.b_slot_ptr[batch], ns = a.b_slot_ptr[batch + 1] - s0;
-    const int c_begin = a.b_chunk_ptr[batch], c_end = a.b_chunk_ptr[batch + 1];
+    const int c_first = a.b_chunk_ptr[batch], nck = a.b_chunk_ptr[batch + 1] - c_first;
+    const int c_begin = c_first + (int)((int64_t)nck * part / parts), c_end = c_first + (int)((int64_t)nck * (part + 1) / parts);
+    Real* const pout = (Real*)a.partials + (parts > 1 ? part * a.n_slots : 0) * d * d + (int64_t)s0 * d * d;
+    Real* const iout = (Real*)a.img_partials + (part * a.n_batches + batch) * a.L * 2 * d;
+    if (c_begin == c_end) {                                                  // fewer chunks than parts: zeros
+        for (int q = tid; q < ns * d * d; q += BA_WAVES * 64) pout[q] = Real(0);
+        for (int q = tid; q < nimg * 2 * d; q += BA_WAVES * 64) iout[q] = Real(0);
+        if (a.work_ctr == nullptr) break;
+        __syncthreads();                 // every wave has read sNext
+        continue;
+    }
     int first_ct = a.chunk_meta[4 * c_begin + 1];
 
     {
@@ -943,7 +956,7 @@ __global__ void __launch_bounds__(BA_WAVES * 64) k_schur(LinArgs a) {
         const int pq = my_pq[q];
         if (pq >= 0) {
             const int sl = my_q[q];
-            Real* P = (Real*)a.partials + (int64_t)(s0 + sl) * d * d;
+            Real* P = pout + (int64_t)sl * d * d;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int i = M::row(lane, v);
@@ -951,7 +964,7 @@ __global__ void __launch_bounds__(BA_WAVES * 64) k_schur(LinArgs a) {
             }
             const int la = pq & 0xff, lb = (pq >> 8) & 0xff;
             if (la == lb && jc == 15) {
-                Real* o = (Real*)a.img_partials + ((int64_t)batch * a.L + la) * 2 * d;
+                Real* o = iout + la * 2 * d;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int i = M::row(lane, v);
@@ -963,7 +976,7 @@ __global__ void __launch_bounds__(BA_WAVES * 64) k_schur(LinArgs a) {
     __syncthreads();
     {
         const int va = tid >> 4, vj = tid & 15;
-        if (va < nimg && vj < d) ((Real*)a.img_partials)[((int64_t)batch * a.L + va) * 2 * d + d + vj] = sDv[va][vj];
+        if (va < nimg && vj < d) iout[va * 2 * d + d + vj] = sDv[va][vj];
     }
     if (a.work_ctr == nullptr) break;
     __syncthreads();                     // this batch's LDS fully read before the next one is staged
@@ -973,6 +986,25 @@ __global__ void __launch_bounds__(BA_WAVES * 64) k_schur(LinArgs a) {
 __global__ void k_ctr_clear(int* ctr) { *ctr = 0; }
 
 // ----------------------------------------------------------------------------- reductions
+// The parts of both partial arrays, added in order into the first part.  A pass of its own: within k_pair_reduce, whose
+// threads walk a pair's batches one after the other, 60 batches of 18 parts took 266 us.
+template <typename Real>
+__global__ void __launch_bounds__(256) k_parts_sum(Real* __restrict__ a, int64_t na, Real* __restrict__ b, int64_t nb,
+                                                   int parts) {
+    int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= na + nb) return;
+    Real* p = t < na ? a + t : b + (t - na);
+    const int64_t n = t < na ? na : nb;
+    Real s = p[0];
+    int h = 1;
+    for (; h + 4 <= parts; h += 4) {                                    // four loads in flight
+        const Real v0 = p[h * n], v1 = p[(h + 1) * n], v2 = p[(h + 2) * n], v3 = p[(h + 3) * n];
+        s += v0; s += v1; s += v2; s += v3;
+    }
+    for (; h < parts; ++h) s += p[h * n];
+    p[0] = s;
+}
+
 template <typename Real>
 __global__ void __launch_bounds__(256) k_pair_reduce(const int* __restrict__ pair_ptr, const int* __restrict__ pair_src,
                                                      const Real* __restrict__ partials, int64_t n_pairs, int d,
@@ -1169,13 +1201,15 @@ static int lin_stage(const ba_lin_args& a, int32_t stage, hipStream_t st) {
     }
     if (stage == 1 && a.n_batches > 0) {
         size_t lds = ((size_t)BA_CHUNK * BA_BLK + 48) * sizeof(Real);
-        // one workgroup per CU (the kernel's LDS allows one) pulling batches from the work queue
-        unsigned grid = (unsigned)a.n_batches;
+        // one workgroup per CU (the kernel's LDS allows one) pulling work items from the queue
+        const int64_t items = a.n_batches * (a.parts > 1 ? a.parts : 1);
+        BA_REQUIRE(items < ((int64_t)1 << 31), "too many parts");
+        unsigned grid = (unsigned)items;
         if (a.work_ctr != nullptr) {
             int dev = 0, n_cu = 0;
             BA_HIP(hipGetDevice(&dev));
             BA_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-            if (n_cu > 0 && (int64_t)n_cu < a.n_batches) grid = (unsigned)n_cu;
+            if (n_cu > 0 && (int64_t)n_cu < items) grid = (unsigned)n_cu;
             hipLaunchKernelGGL(k_ctr_clear, dim3(1), dim3(1), 0, st, a.work_ctr);
         }
         BA_DISPATCH_KP(a.lay, {
@@ -1183,6 +1217,11 @@ static int lin_stage(const ba_lin_args& a, int32_t stage, hipStream_t st) {
                                        (int)lds));
             hipLaunchKernelGGL((k_schur<HK_, HP_, Real>), dim3(grid), dim3(BA_WAVES * 64), lds, st, a);
         });
+        if (a.parts > 1) {
+            const int64_t na = a.n_slots * a.lay.d * a.lay.d, nb = a.n_batches * a.L * 2 * a.lay.d;
+            hipLaunchKernelGGL(k_parts_sum<Real>, dim3(nblk(na + nb, 256)), dim3(256), 0, st, (Real*)a.partials, na,
+                               (Real*)a.img_partials, nb, (int)a.parts);
+        }
         BA_LAUNCHED();
     }
     if (stage == 1) return BA_OK;
@@ -1198,6 +1237,28 @@ static int lin_stage(const ba_lin_args& a, int32_t stage, hipStream_t st) {
     return BA_OK;
 }
 
+// k_schur runs one work item per CU at a time.  A batch is as long as its 96 pair slots allow, so a reconstruction of a
+// few hundred images has fewer batches than the chip has CUs, or one and a bit per CU.  In chunks (about 7 us each in
+// fp64): the items go round in ceil(items / CUs) turns of an average part and half a chunk of start and flush, or take
+// as long as the longest; writing, adding and reading an item's partials costs 0.006.  At most 8 items per CU, so the
+// partials stay below 2048 x 96 blocks.  Measured, k_schur + reductions in us at 1 part / here: 8 images 1 batch 105 + 11
+// / 17 + 12, 14 images 60 batches 961 + 26 / 73 + 73, 200 images 95 batches 548 + 20 / 175 + 24 (4 parts 201 + 23, 6:
+// 203 + 25, 8: 175 + 30), 400 images 195 batches 450 + 15 / 279 + 38, 777 images fp32 383 batches 1469 + 21 / 1183 + 33;
+// 507 batches (2 parts: 2309 + 25 -> 2249 + 54) and 1245 (2348 + 46 -> 2326 + 130) stay whole.
+extern "C" int32_t ba_schur_parts(int64_t n_batches, int64_t n_chunks, int64_t max_chunks, int32_t n_cu) {
+    if (n_batches < 1 || n_chunks < 1 || max_chunks < 1 || n_cu < 1) return 1;
+    const double avg = (double)n_chunks / (double)n_batches;
+    double best = INFINITY;
+    int32_t pick = 1;
+    for (int64_t p = 1; p <= max_chunks && p <= INT32_MAX && (p == 1 || p * n_batches <= 8 * (int64_t)n_cu); ++p) {
+        const int64_t items = p * n_batches, turns = (items + n_cu - 1) / n_cu;
+        const double mean = (double)turns * (avg / (double)p + 0.5), most = (double)max_chunks / (double)p + 0.5;
+        const double cost = (mean > most ? mean : most) + 0.006 * (double)items;
+        if (cost < best) { best = cost; pick = (int32_t)p; }
+    }
+    return pick;
+}
+
 extern "C" int ba_linearize_stage(const ba_lin_args* args, int32_t stage, void* stream) {
     clear_error();
     BA_REQUIRE(args != nullptr, "null args");
@@ -1211,6 +1272,7 @@ extern "C" int ba_linearize_stage(const ba_lin_args* args, int32_t stage, void* 
     BA_REQUIRE(a.L >= 1 && a.L <= BA_MAX_LOCAL, "bad plan L");
     BA_REQUIRE(stage >= 0 && stage <= 2, "stage must be 0, 1 or 2");
     BA_REQUIRE(a.real32 == 0 || a.real32 == 1, "real32 must be 0 or 1");
+    BA_REQUIRE(a.parts <= 1 || a.n_slots >= 0, "bad part count");
     if (a.n_chunks > 0) {
         const char* miss = missing_pointer(a, stage);
         BA_REQUIRE(miss == nullptr, miss);

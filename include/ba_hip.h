@@ -164,7 +164,16 @@ typedef struct {
      * dtype=torch.float32 default, ba_solver.py:22, :37, :128): the Jacobian core and the weighted rows of
      * an observation are evaluated in fp64 and rounded, every product, sum and factor after them is fp32 */
     int32_t real32;
+    /* parts > 1: stage 1 cuts each batch's chunks into that many parts, each a work item with partials of its own, and
+     * adds the parts in order into the first; partials is then (parts, n_slots, d, d) and img_partials (parts,
+     * n_batches, L, 2, d).  0 or 1: whole batches, (n_slots, d, d) and (n_batches, L, 2, d) */
+    int32_t parts;
+    int64_t n_slots;         /* plan: BA_PS_N_SLOTS (read when parts > 1) */
 } ba_lin_args;
+
+/* parts (1 .. max_chunks) of each batch that spread n_batches batches of n_chunks chunks together, max_chunks at most,
+ * best over n_cu compute units */
+int32_t ba_schur_parts(int64_t n_batches, int64_t n_chunks, int64_t max_chunks, int32_t n_cu);
 
 /* Stages 1-3: point blocks, camera-pair Schur blocks, rhs and diag(H_cc) at image level.
  * Requires d <= 15 and C <= 24. */
