@@ -8,10 +8,12 @@ computed: ``compute_jacobians`` returns a light handle instead of materialised
 fp64 Jacobian blocks, and ``solve_delta`` runs the fused HIP path
 
     ba_linearize_schur   J, J^T W r, H_pp, camera-pair blocks of S, rhs (fp64, on chip)
-    ba_pcg_solve         the reference's Jacobi-PCG (bs:184-206, :1197-1238) on the explicit S
+    ba_pcg_solve*        the reference's Jacobi-PCG (bs:184-206, :1197-1238) on the explicit S: resident in one
+                         launch, by pair blocks, or two launches per iteration
     ba_backsubstitute    delta_p = H_pp^-1 (g_p - H_pc delta_c)
 
-with no host synchronisation between them.
+with no host synchronisation between them; after a resident solve the host reads its outcome (8 words) once the
+back-substitution is enqueued.
 """
 import ctypes
 

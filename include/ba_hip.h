@@ -429,7 +429,7 @@ int ba_apply_update(const float* K, const float* P_w2rig, const float* z_coefs, 
                     int32_t n_cams, int32_t n_nodes, int32_t n_imgs, int32_t C, int64_t n_tracks, float* K_out,
                     float* P_out, float* z_out, float* X_out, void* stream);
 
-/* Bytes of device workspace ba_objective needs for n_obs observations. */
+/* Bytes of device workspace ba_objective needs for n_obs observations (4 per observation and 76 KB). */
 int64_t ba_objective_workspace_bytes(int64_t n_obs);
 
 /* Line-search objective of lm_step (engine.py:263-278, :357-361) from the residual buffer of
@@ -441,8 +441,8 @@ int ba_objective(const float* res, int64_t n_obs, int32_t has_err, void* workspa
 /* ba_objective without a workspace argument and without any allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  The passes recompute each observation's
- * key from res instead of storing it, and keep their partial sums (at most 2048 blocks) in a static
- * per-GPU scratch array of 42 KB, so every n_obs fits (up to the 32-bit rank limit that
+ * key from res instead of storing it, and keep their partial sums (at most 512 blocks) and counters in a static
+ * per-GPU scratch array of 76 KB, so every n_obs fits (up to the 32-bit rank limit that
  * ba_objective shares: n_obs <= 5368709119, rejected with an error beyond).  Outputs equal
  * ba_objective's bit for bit.  All calls on one GPU share its scratch array: calls that overlap on
  * one GPU (other streams, other threads) race and must be serialised by the caller. */
