@@ -948,6 +948,8 @@ __global__ void __launch_bounds__(PCG_T) k_pp_clear(uint64_t* __restrict__ w, in
     if (t < 8) istate[t] = 0;
 }
 
+__global__ void k_pp_refused(int32_t* istate) { istate[6] = 1; }
+
 // DM: the block width the product is unrolled for (d <= DM <= GW); NS: shared unknowns exchanged.  The first
 // wave owns the workgroup's entries (their x, r, z, p and the loop's partial sums); all waves poll, form the
 // loop's scalars and take part in the product.  Four barriers per iteration.
@@ -1477,7 +1479,17 @@ static int resident_launch(ba_pcg_args a, ba_pcg_resident w, hipStream_t st) {
     hipLaunchKernelGGL(k_leaf_damp<Real>, dim3(nb), dim3(PCG_T), 0, st, a);
     BA_LAUNCHED();
     void* args[] = {&a, &w};
-    BA_HIP(hipLaunchCooperativeKernel(k, dim3((unsigned)((a.n_imgs + w.m - 1) / w.m)), dim3(PP_T), args, (unsigned)lds, st));
+    const hipError_t e = hipLaunchCooperativeKernel(k, dim3((unsigned)((a.n_imgs + w.m - 1) / w.m)), dim3(PP_T), args,
+                                                    (unsigned)lds, st);
+    if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
+        // fewer CUs than the device reports (a process with a CU mask), or no cooperative launches: as after a
+        // wait that gave up
+        (void)hipGetLastError();
+        hipLaunchKernelGGL(k_pp_refused, dim3(1), dim3(1), 0, st, a.istate);
+        BA_LAUNCHED();
+        return BA_OK;
+    }
+    BA_HIP(e);
     return BA_OK;
 }
 

@@ -195,11 +195,11 @@ int ba_backsubstitute(const ba_lin_args* args, void* stream);
  * d <= 15, tracks within 13 images and 128 observations, and is slow on random co-visibility).
  * Structure from ba_pm_plan_create (host) or ba_pm_dplan_create (device); a run is the observations of
  * one track in one image:
- *   per observation       J_p^T J_p and J_p^T W r (pobs); per wave of BA_PM_SPAN observations and
+ *   per observation       J_p^T J_p and J_p^T W r (pobs); per wave of 64 to BA_PM_SPAN observations and
  *                         image, sum J_c^T J_c and J_c^T W r (jslots, MFMA)
  *   per track             H_pp, g_p in image order; the point-leaf damping; L, L^-1 g_p
- *   per run (t, i)        V_ti = (sum J_c^T J_p) L^-T (V, 3 x dp per run); per wave of BA_PM_SPAN
- *                         runs and image, sum V V^T and V L^-1 g_p (vslots, MFMA)
+ *   per run (t, i)        V_ti = (sum J_c^T J_p) L^-T (V, 3 x dp per run); per wave of 64 to
+ *                         BA_PM_SPAN runs and image, sum V V^T and V L^-1 g_p (vslots, MFMA)
  *   per image i           S_ii, rhs and diag(H_cc) from its slots, summed in wave order
  *   per image pair (i, j) S_ij = - sum_t V_ti V_tj^T over the pair's terms (one wave, MFMA)
  * Replaces the same reference work as ba_linearize_schur (ba_solver.py:110-206). */
@@ -349,8 +349,8 @@ int ba_pcg_solve_pairs_range(const ba_pcg_args* args, const ba_pcg_pairs* pairs,
 /* The same solve in one cooperative launch, each workgroup holding m image rows in LDS and exchanging partial
  * sums and z with the others through `words` (for systems whose rows fit and at most 2 unknowns that several
  * image-level entries share; the unknowns' lists must ascend, as the planners make them).  istate[6] is set,
- * and x not, when a wait exceeded `limit`: solve with ba_pcg_solve then.  Of the workspace of args it uses rhs,
- * diagA, damp, x, state and istate only.  Not for capture into a graph. */
+ * and x not, when a wait exceeded `limit` or the device refused the launch: solve with ba_pcg_solve then.  Of the
+ * workspace of args it uses rhs, diagA, damp, x, state and istate only.  Not for capture into a graph. */
 typedef struct {
     uint64_t* words;                   /* ba_pcg_resident_words(...) words of workspace */
     const int32_t* shared_u;           /* (n_shared) the unknowns with two or more image-level entries, all of them */
