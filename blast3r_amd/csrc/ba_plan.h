@@ -105,5 +105,5 @@ enum {
                             //   without terms last
     BA_PM_NARRAYS
 };
-#define BA_PM_SPAN 512        // observations (runs) per wave of the pair-major per-image sums
+#define BA_PM_SPAN 512        // most observations (runs) per wave of the pair-major per-image sums
 enum { BA_PMS_N_RUNS = 0, BA_PMS_N_PAIRS, BA_PMS_N_TERMS, BA_PMS_MAX_TERMS, BA_PMS_MAX_TRACK_RUNS, BA_PM_NSCALARS };

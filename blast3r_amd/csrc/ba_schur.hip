@@ -1308,12 +1308,29 @@ extern "C" int ba_backsubstitute(const ba_lin_args* args, void* stream) {
 namespace ba {
 
 #define PM_T 256
-#define PM_SPAN BA_PM_SPAN  // observations (runs) per wave of k_pm_obs (k_pm_runs)
+#define PM_WAVES 8192       // waves up to which spans are halved
+// Observations (runs) per wave of k_pm_obs (k_pm_runs), from their number: 64 to BA_PM_SPAN.  The chip holds 1536 to
+// 3072 of these waves; with fewer it idles, with a few times as many the last ones still run alone, and each round
+// of 64 is a chain of loads, Jacobians and a serial sum.  A wave more costs a slot (1 or 3 tiles of 256 values written
+// and read back by k_pm_diag) per image that it meets.  Linearise + Schur in us, spans of 512 throughout / halved up to
+// 2048 waves / 4096 / 8192 / 16384:
+//   d = 13, 110 k observations   fp64  262 / 125 / 125 / 125 / 125       fp32  190 /  84 /  84 /  84 /  84
+//           60 k                       272 / 114 / 115 / 115 / 115             202 /  92 /  92 /  91 /  92
+//           600 k                      561 / 509 / 514 / 508 / 509             362 / 338 / 315 / 310 / 309
+//           1.3 M                      941 / 940 / 949 / 927 / 948             627 / 626 / 583 / 559 / 575
+//           3.25 M                     2308 / 2300 / 2308 / 2202 / 2175        1446 / 1435 / 1438 / 1377 / 1354
+//   d = 23, 150 k                      502 / 337 / 336 / 337 / 338             341 / 207 / 208 / 207 / 207
+//           1.3 M                      2133 / 2135 / 2054 / 2029 / 2079        1157 / 1153 / 1157 / 1119 / 1161
+__host__ __device__ inline int pm_span(int64_t n_items) {
+    int span = BA_PM_SPAN;
+    while (span > 64 && n_items < (int64_t)span * PM_WAVES) span >>= 1;
+    return span;
+}
 // waves of k_pm_obs sharing one staging buffer: two in fp64 (the buffer, not the registers, limited
 // the CU to 1.5 waves per SIMD; measured at config 3: 17.33 -> 17.05 ms per pass), one in fp32 (the
 // registers already allow no more waves than buffers; two waves there cost 3.5% in their turns)
 template <typename Real> struct PmObsWaves { static constexpr int N = sizeof(Real) == 8 ? 2 : 1; };
-static_assert(PM_SPAN % 64 == 0, "a span is whole rounds of 64 observations");
+static_assert(BA_PM_SPAN % 64 == 0 && (BA_PM_SPAN & (BA_PM_SPAN - 1)) == 0, "a span is whole rounds of 64 observations");
 
 typedef ba_pm_args PmArgs;
 
@@ -1468,7 +1485,7 @@ struct PmTileAcc {
     }
 };
 
-// Per observation (one wave per PM_SPAN observations, 64 at a time): J_p^T J_p (upper 6) and
+// Per observation (one wave per pm_span observations, 64 at a time): J_p^T J_p (upper 6) and
 // J_p^T W r (3) to pobs, sqrt(W) to wobs; the weighted camera rows, with sqrt(W) r in column d,
 // staged in LDS and summed per image (X^T X) into the J slots.  PmObsWaves waves share one staging
 // buffer and take turns with it: each wave linearises its observations of a round in registers (the
@@ -1482,13 +1499,14 @@ __global__ void __launch_bounds__(64 * PmObsWaves<Real>::N, 3) k_pm_obs(PmArgs a
     __shared__ int simg[64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int64_t w = (int64_t)blockIdx.x * NW + wv;
-    const int64_t o_begin = w * PM_SPAN, o_end = min(o_begin + PM_SPAN, a.n_obs);   // empty past the end
+    const int span = pm_span(a.n_obs);
+    const int64_t o_begin = w * span, o_end = min(o_begin + span, a.n_obs);   // empty past the end
     const int d = a.lay.d;
     PmTileAcc<DP, Real> T;
     T.img = -1;
     T.zero();
 #pragma unroll 1
-    for (int rnd = 0; rnd < PM_SPAN / 64; ++rnd) {     // the same rounds in every wave (barriers below)
+    for (int rnd = 0; rnd < span / 64; ++rnd) {     // the same rounds in every wave (barriers below)
         const int64_t o = o_begin + 64 * rnd + lane;
         int img = -1;
         ObsCtx c;
@@ -1607,7 +1625,7 @@ __global__ void __launch_bounds__(256) k_pm_factor(PmArgs a, const Real* __restr
     for (int e = threadIdx.x; e < nt * NV; e += 256) dst[e] = rec[(e / NV) * STR + e % NV];
 }
 
-// Per run (one wave per PM_SPAN runs, 64 at a time): V = sum over the run's observations of
+// Per run (one wave per pm_span runs, 64 at a time): V = sum over the run's observations of
 // sum_R jc_R (L^-1 jp_R)^T (= (sum J_c^T J_p) L^-T), staged in LDS with L^-1 g_p in column d,
 // summed per image (-X^T X) into the V slots and copied to V (run-major, 3 x DP per run).
 template <int HK, int HP, int DP, typename Real>
@@ -1616,7 +1634,8 @@ __global__ void __launch_bounds__(64, 2) k_pm_runs(PmArgs a) {
     __shared__ int simg[64];
     const int lane = threadIdx.x;
     const int64_t w = blockIdx.x;
-    const int64_t r_begin = w * PM_SPAN, r_end = min(r_begin + PM_SPAN, a.n_runs);
+    const int span = pm_span(a.n_runs);
+    const int64_t r_begin = w * span, r_end = min(r_begin + span, a.n_runs);
     const int d = a.lay.d;
     PmTileAcc<DP, Real> T;
     T.img = -1;
@@ -1705,6 +1724,21 @@ __global__ void __launch_bounds__(64, 2) k_pm_runs(PmArgs a) {
     if (T.img >= 0) T.flush((Real*)a.vslots, w, lane);
 }
 
+// s += entry e of the slots first .. last, in order, 8 loads in flight
+template <int NTL, typename Real>
+__device__ __forceinline__ void pm_slots_sum(const Real* __restrict__ slots, int64_t first, int64_t last, int e, Real& s) {
+    const Real* p = slots + first * (NTL * 256) + e;
+    int64_t n = last - first + 1;
+    for (; n >= 8; n -= 8, p += 8 * NTL * 256) {
+        Real v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = p[k * NTL * 256];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s += v[k];
+    }
+    for (; n > 0; --n, p += NTL * 256) s += *p;
+}
+
 // Per image i: the J and V slots of the waves that held its observations and runs, summed in wave
 // order: S_ii (lower tiles, mirrored), rhs_i (row d) and diag(H_cc)_i (the J part's diagonal).
 template <int DP, typename Real>
@@ -1720,14 +1754,15 @@ __global__ void __launch_bounds__(256) k_pm_diag(PmArgs a) {
     }
     const int64_t o0 = i ? a.infos[i - 1] : 0, o1 = a.infos[i];
     const int64_t r0 = a.img_run_ptr[i], r1 = a.img_run_ptr[i + 1];
-    const int64_t wj0 = o0 / PM_SPAN, wj1 = (o1 - 1) / PM_SPAN, wv0 = r0 / PM_SPAN, wv1 = (r1 - 1) / PM_SPAN;
+    const int so = pm_span(a.n_obs), sr = pm_span(a.n_runs);
+    const int64_t wj0 = o0 / so, wj1 = (o1 - 1) / so, wv0 = r0 / sr, wv1 = (r1 - 1) / sr;
     Real* S = (Real*)a.S_pairs + (int64_t)pd * d * d;
     const Real* jslots = (const Real*)a.jslots;
     const Real* vslots = (const Real*)a.vslots;
     for (int e = t; e < NTL * 256; e += 256) {
         Real sj = Real(0), sv = Real(0);
-        for (int64_t w = wj0; w <= wj1; ++w) sj += jslots[(w + i) * (NTL * 256) + e];
-        for (int64_t w = wv0; w <= wv1; ++w) sv += vslots[(w + i) * (NTL * 256) + e];
+        pm_slots_sum<NTL>(jslots, wj0 + i, wj1 + i, e, sj);
+        pm_slots_sum<NTL>(vslots, wv0 + i, wv1 + i, e, sv);
         const int q = e >> 8, ri = (e >> 4) & 15, cj = e & 15;
         int hi = 0, hj = 0, qq = 0;
 #pragma unroll
@@ -1970,7 +2005,7 @@ static void pm_stage(const ba_pm_args& a, int stage, hipStream_t st) {
     Real* const lam_p = (Real*)a.lam_p;
     hipLaunchKernelGGL(k_lam_clear<Real>, dim3(1), dim3(1), 0, st, tmax, nbt);
     if (a.n_obs > 0) {
-        const int64_t nw = (a.n_obs + PM_SPAN - 1) / PM_SPAN;          // waves (spans of PM_SPAN observations)
+        const int64_t span = pm_span(a.n_obs), nw = (a.n_obs + span - 1) / span;        // waves, one per span
         constexpr int NW = PmObsWaves<Real>::N;
         const unsigned g = (unsigned)((nw + NW - 1) / NW);
         BA_DISPATCH_KP(a.lay, {
@@ -1988,7 +2023,8 @@ static void pm_stage(const ba_pm_args& a, int stage, hipStream_t st) {
     if (a.n_tracks > 0)
         hipLaunchKernelGGL(k_pm_factor<Real>, dim3(nblk(a.n_tracks, 256)), dim3(256), 0, st, a, (const Real*)lam_p);
     if (a.n_runs > 0) {
-        const unsigned g = (unsigned)((a.n_runs + PM_SPAN - 1) / PM_SPAN);
+        const int64_t span = pm_span(a.n_runs);
+        const unsigned g = (unsigned)((a.n_runs + span - 1) / span);
         BA_DISPATCH_KP(a.lay, {
             if (wide) hipLaunchKernelGGL((k_pm_runs<HK_, HP_, 32, Real>), dim3(g), dim3(64), 0, st, a);
             else      hipLaunchKernelGGL((k_pm_runs<HK_, HP_, 16, Real>), dim3(g), dim3(64), 0, st, a);
@@ -2010,7 +2046,8 @@ static void pm_backsub(const ba_pm_args& a, hipStream_t st) {
 extern "C" int64_t ba_pm_slot_doubles(int64_t n_items, int32_t n_imgs, int32_t d) {
     if (n_items < 0 || n_imgs < 0 || d < 1 || d > 31) return -1;
     const int64_t ntl = d < 16 ? 1 : 3;
-    return ((n_items + PM_SPAN - 1) / PM_SPAN + n_imgs) * ntl * 256;
+    const int64_t span = pm_span(n_items);
+    return ((n_items + span - 1) / span + n_imgs) * ntl * 256;
 }
 
 extern "C" int ba_pm_linearize_stage(const ba_pm_args* args, int stage, void* stream) {
