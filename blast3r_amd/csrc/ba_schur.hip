@@ -2042,12 +2042,17 @@ static void pm_backsub(const ba_pm_args& a, hipStream_t st) {
         hipLaunchKernelGGL((k_pm_backsub<16, Real>), dim3(nblk(a.n_tracks, 256 / 16)), dim3(256), 0, st, a);
 }
 
-// elements (of the working precision) of one slot array
+// Elements (of the working precision) of one slot array: a slot per wave and per image.  Fewer items can take shorter
+// spans and so more waves (2^20 - 1 items 16384 waves, 2^20 items 8192): the size is the most that any number of items
+// up to n_items needs, so that an array sized for the largest call holds every smaller one.
 extern "C" int64_t ba_pm_slot_doubles(int64_t n_items, int32_t n_imgs, int32_t d) {
     if (n_items < 0 || n_imgs < 0 || d < 1 || d > 31) return -1;
     const int64_t ntl = d < 16 ? 1 : 3;
     const int64_t span = pm_span(n_items);
-    return ((n_items + span - 1) / span + n_imgs) * ntl * 256;
+    int64_t waves = (n_items + span - 1) / span;
+    // a span s gives way to 2 s at 2 s PM_WAVES items, where it had reached 2 PM_WAVES waves
+    if (span > 64 && waves < 2 * PM_WAVES) waves = 2 * PM_WAVES;
+    return (waves + n_imgs) * ntl * 256;
 }
 
 extern "C" int ba_pm_linearize_stage(const ba_pm_args* args, int stage, void* stream) {

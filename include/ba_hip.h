@@ -267,8 +267,8 @@ int ba_pm_linearize_schur(const ba_pm_args* args, void* stream);
 /* the same in two launches sequences: stage 0 = observations, tracks, damping, point factors, runs and
  * per-image blocks; stage 1 = the off-diagonal pair blocks (k_pm_pairs), for timing them apart */
 int ba_pm_linearize_stage(const ba_pm_args* args, int stage, void* stream);
-/* doubles of one slot array of ba_pm_args (n_items = n_obs for jslots, n_runs for vslots); -1 for d
- * outside 1..31 */
+/* Elements (R) of one slot array of ba_pm_args (n_items = n_obs for jslots, n_runs for vslots); -1 for d outside
+ * 1..31.  Never smaller for more items or images: an array of this size also serves every call with fewer. */
 int64_t ba_pm_slot_doubles(int64_t n_items, int32_t n_imgs, int32_t d);
 /* delta_p = L^-T (L^-1 g_p - sum_i V_ti^T delta_c(i)) per track (= (H_pp + lam_p I)^-1 (g_p - H_pc delta_c)) */
 int ba_pm_backsubstitute(const ba_pm_args* args, void* stream);
