@@ -349,8 +349,9 @@ int ba_pcg_solve_pairs_range(const ba_pcg_args* args, const ba_pcg_pairs* pairs,
 /* The same solve in one cooperative launch, each workgroup holding m image rows in LDS and exchanging partial
  * sums and z with the others through `words` (for systems whose rows fit and at most 2 unknowns that several
  * image-level entries share; the unknowns' lists must ascend, as the planners make them).  istate[6] is set,
- * and x not, when a wait exceeded `limit` or the device refused the launch: solve with ba_pcg_solve then.  Of the
- * workspace of args it uses rhs, diagA, damp, x, state and istate only.  Not for capture into a graph. */
+ * and x not, when a wait exceeded `limit`, the device refused the launch, or max_blk or max_col is less than the rows
+ * need: solve with ba_pcg_solve then.  Of the workspace of args it uses rhs, diagA, damp, x, state and istate only.
+ * Not for capture into a graph. */
 typedef struct {
     uint64_t* words;                   /* ba_pcg_resident_words(...) words of workspace */
     const int32_t* shared_u;           /* (n_shared) the unknowns with two or more image-level entries, all of them */

@@ -247,6 +247,35 @@ def test_resident_solve(m, d, shared, per, real32):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('m,d,shared', [(7, 13, 2), (61, 10, 2), (250, 13, 2), (33, 17, 2)])
+def test_resident_solve_with_sizes_too_small(m, d, shared):
+    """max_blk or max_col one less than the rows need: the kernel gives up before it writes either array, in whichever
+    workgroups it is too little for (the others' waits end at their limit); with exactly what they need, the plan's
+    solve bit for bit."""
+    from blast3r_amd._lib import check, lib, stream_ptr
+    sysm = block_system(m, d, shared, seed=m * 100 + d, density=0.6 if m < 100 else 0.04)
+    pa, keep = pcg_args(sysm, 8, 0.0, False)
+    res, hold = resident_args(sysm, pa)
+    blk, per = res.max_blk, res.m
+    cols = lambda g: {x for i, j in sysm['pairs'] for x in (i, j) if g[0] <= i < g[1] or g[0] <= j < g[1]} | set(range(*g))
+    col = max(len(cols((i, min(i + per, m)))) for i in range(0, m, per))
+    solve = lambda: check(lib().ba_pcg_solve_resident(ctypes.byref(pa), ctypes.byref(res), stream_ptr(DEV)))
+    solve()
+    x = keep['x'].clone()
+    res.limit = 1_000_000                              # 10 ms
+    for max_blk, max_col in ((blk, col - 1), (blk - 1, col), (blk, 1), (1, col), (blk, col)):
+        few = (max_blk < blk and blk > 1) or max_col < col
+        if max_blk < 1:
+            continue
+        print(f'resident sizes m={m} d={d} blk={max_blk} of {blk} col={max_col} of {col}', flush=True)
+        res.max_blk, res.max_col = max_blk, max_col
+        keep['x'].zero_()
+        solve()
+        assert bool(keep['istate'][6]) == few
+        assert few or torch.equal(keep['x'], x)
+
+
+@pytest.mark.gpu
 def test_resident_solve_gives_up_and_the_launch_sequence_takes_over(monkeypatch):
     """A resident loop whose waits are limited to nothing leaves at once, says so, and solve_delta returns the launch
     sequence's step; with the usual limit it returns the same step to rounding."""
