@@ -1272,7 +1272,7 @@ extern "C" int ba_linearize_stage(const ba_lin_args* args, int32_t stage, void* 
     BA_REQUIRE(a.L >= 1 && a.L <= BA_MAX_LOCAL, "bad plan L");
     BA_REQUIRE(stage >= 0 && stage <= 2, "stage must be 0, 1 or 2");
     BA_REQUIRE(a.real32 == 0 || a.real32 == 1, "real32 must be 0 or 1");
-    BA_REQUIRE(a.parts <= 1 || a.n_slots >= 0, "bad part count");
+    BA_REQUIRE(a.parts <= 1 || a.n_slots >= (a.n_chunks > 0 ? 1 : 0), "bad part count, or parts without n_slots");
     if (a.n_chunks > 0) {
         const char* miss = missing_pointer(a, stage);
         BA_REQUIRE(miss == nullptr, miss);

@@ -168,7 +168,7 @@ typedef struct {
      * adds the parts in order into the first; partials is then (parts, n_slots, d, d) and img_partials (parts,
      * n_batches, L, 2, d).  0 or 1: whole batches, (n_slots, d, d) and (n_batches, L, 2, d) */
     int32_t parts;
-    int64_t n_slots;         /* plan: BA_PS_N_SLOTS (read when parts > 1) */
+    int64_t n_slots;         /* plan: BA_PS_N_SLOTS (needed when parts > 1) */
 } ba_lin_args;
 
 /* parts (1 .. max_chunks) of each batch that spread n_batches batches of n_chunks chunks together, max_chunks at most,

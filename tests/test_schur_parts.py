@@ -23,6 +23,22 @@ def test_parts_rule():
                 assert 1 <= p <= most and (p == 1 or p * nb <= 8 * 256)
 
 
+def test_parts_need_the_slot_count():
+    """Parts whose partials would all begin at the same place are refused on the host (before any pointer is looked at)."""
+    from blast3r_amd._lib import BaLinArgs, lib
+    a = BaLinArgs()
+    a.L, a.n_chunks, a.n_batches = 4, 4, 2
+    a.lay.d, a.lay.C, a.lay.off_tau, a.lay.off_zcf, a.lay.hasK, a.lay.hasP, a.lay.hasZ = 13, 5, 2, 8, 1, 1, 1
+    for parts, n_slots, msg in ((2, 0, b'part count'), (2, -1, b'part count'), (2, 3, b'null pointer'),
+                                (1, 0, b'null pointer'), (0, 0, b'null pointer')):
+        a.parts, a.n_slots = parts, n_slots
+        for call in (lambda: lib().ba_linearize_schur(ctypes.byref(a), None),
+                     lambda: lib().ba_linearize_stage(ctypes.byref(a), 1, None)):
+            assert call() != 0 and msg in lib().ba_last_error(), (parts, n_slots)
+    a.parts, a.n_slots, a.n_chunks, a.n_batches = 2, -1, 0, 0
+    assert lib().ba_linearize_stage(ctypes.byref(a), 1, None) != 0 and b'part count' in lib().ba_last_error()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('dtype', [torch.float64, torch.float32], ids=['fp64', 'fp32'])
 @pytest.mark.parametrize('cfg,nf,nt,flags', [(0, 8, 40, {}), (0, 8, 300, {}), (2, 24, 800, {}), (2, 60, 6000, {}),
