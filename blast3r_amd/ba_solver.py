@@ -16,6 +16,7 @@ with no host synchronisation between them; after a resident solve the host reads
 back-substitution is enqueued.
 """
 import ctypes
+import threading
 
 import numpy as np
 import torch
@@ -90,7 +91,39 @@ def _flag(status, name, count, device):
 # fp32, with 18 M 2.3 and 2.5 us faster, with 37 M 9.2 and 7.9 us, with 188 M 108 and 93 us
 PCG_ROWS_MOST = 14_000_000
 RESIDENT_LIMIT = 10_000_000     # longest wait inside the resident solve, in ticks of 10 ns
+RESIDENT_GIVE_UPS = 3           # waits in vain in a row after which a device's solves go by launches ...
+RESIDENT_RETRY = 64             # ... all but one after this many, after twice as many once that waits in vain too, ...
+RESIDENT_RETRY_MOST = 4096      # ... up to this many
 PCG_CHUNK = 25          # PCG iterations per graph when the host stops launching after the loop stops
+
+
+class _GiveUps:
+    """Resident solves of one device that gave up waiting, in a row.  While another process holds CUs every resident
+    solve waits RESIDENT_LIMIT in vain (0.1 s, against some 5 ms by launches), and in an online reconstruction each added
+    frame is a structure that has not been tried yet."""
+    _of, _lock = {}, threading.Lock()
+
+    def __init__(self):
+        self.n, self.skip = 0, 0
+
+    @classmethod
+    def of(cls, device):
+        index = torch.cuda.current_device() if device.index is None else device.index
+        with cls._lock:
+            return cls._of.setdefault(index, cls())
+
+    def try_now(self):
+        """Whether the next solve may be resident."""
+        with self._lock:
+            if self.n < RESIDENT_GIVE_UPS:
+                return True
+            self.skip -= 1
+            return self.skip < 0
+
+    def outcome(self, gave_up):
+        with self._lock:
+            self.n = self.n + 1 if gave_up else 0
+            self.skip = min(RESIDENT_RETRY << min(max(self.n - RESIDENT_GIVE_UPS, 0), 16), RESIDENT_RETRY_MOST)
 
 
 class GaussNewtonSolver:
@@ -654,8 +687,9 @@ class GaussNewtonSolver:
     def _run_resident(self, pa, um, plan, st):
         """Enqueues ba_pcg_solve_resident (the whole loop in one launch) where it applies: rows that fit the
         workgroups' registers and LDS, few shared unknowns, no capture under way, and no resident solve of this
-        structure that gave up waiting (as when another process holds part of the GPU).  Returns whether it was
-        launched; its outcome is read by _resident_status once the back-substitution is enqueued too."""
+        structure, or several in a row of the device, that gave up waiting (as when another process holds part of the
+        GPU).  Returns whether it was launched; its outcome is read by _resident_status once the back-substitution is
+        enqueued too."""
         if pa.maxiter < 1 or torch.cuda.is_current_stream_capturing():
             return False
         sizes = um.get(('resident', pa.real32))
@@ -667,7 +701,7 @@ class GaussNewtonSolver:
                                            um['n_shared'], n_cu, ctypes.byref(blk), ctypes.byref(col))
             sizes = um[('resident', pa.real32)] = (m, blk.value, col.value)
         m, max_blk, max_col = sizes
-        if m < 1:
+        if m < 1 or not _GiveUps.of(self.device).try_now():
             return False
         L = lib()
         nw = int(L.ba_pcg_resident_words(pa.n_imgs, pa.d, pa.real32, m))
@@ -678,8 +712,9 @@ class GaussNewtonSolver:
 
     def _resident_status(self, istate, um, pa):
         """The resident solve's outcome (one read per solve): False when it gave up waiting, which keeps this
-        structure to the launch sequence from then on."""
+        structure to the launch sequence from then on, and after a few in a row the device's other ones for a while."""
         ist = istate.tolist()
+        _GiveUps.of(self.device).outcome(bool(ist[6]))
         if ist[6]:
             um[('resident', pa.real32)] = (0, 0, 0)
             return False

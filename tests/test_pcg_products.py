@@ -295,3 +295,44 @@ def test_resident_solve_gives_up_and_the_launch_sequence_takes_over(monkeypatch)
         steps[limit] = info['delta']
     a, b = steps.values()
     assert torch.isfinite(a).all() and float((a - b).norm() / b.norm()) < 1e-4
+
+
+def test_a_device_whose_resident_solves_give_up_is_left_to_the_launches(monkeypatch):
+    """New structures, as an online reconstruction makes them, on a device whose CUs another process holds: after three
+    waits in vain the device's solves go by launches, with a try now and then, and back once one succeeds; other devices
+    are not concerned.  The library is a stub, so that this runs anywhere."""
+    from types import SimpleNamespace
+
+    from blast3r_amd import ba_solver
+    stub = SimpleNamespace(ba_pcg_resident_plan=lambda *a: 1, ba_pcg_resident_words=lambda *a: 8,
+                           ba_pcg_solve_resident=lambda *a: 0)
+    monkeypatch.setattr(ba_solver, 'lib', lambda: stub)
+    monkeypatch.setattr(ba_solver, 'ptr', lambda t: t.data_ptr())
+    monkeypatch.setattr(torch.cuda, 'is_current_stream_capturing', lambda: False)
+    monkeypatch.setattr(torch.cuda, 'get_device_properties', lambda d: SimpleNamespace(multi_processor_count=256))
+    pa = SimpleNamespace(maxiter=300, n_imgs=4, d=3, real32=0)
+    plan = SimpleNamespace(host=dict(row_ptr=np.arange(5, dtype=np.int32)),
+                           workspace=lambda name, shape, dtype: torch.zeros(shape, dtype=dtype))
+
+    def solves(device, n, gave_up, um=None):
+        """The number of n solves, each of a new structure (or of um), that waited."""
+        tries = 0
+        for _ in range(n):
+            s = ba_solver.GaussNewtonSolver(1, 4, 4, 10, device)
+            u = dict(n_shared=0, shared_u=torch.zeros(1, dtype=torch.int32)) if um is None else um
+            if s._run_resident(pa, u, plan, None):
+                tries += 1
+                assert s._resident_status(torch.tensor([0, 0, 5, 1, 5, 0, int(gave_up), 0]), u, pa) != gave_up
+        return tries
+
+    one = dict(n_shared=0, shared_u=torch.zeros(1, dtype=torch.int32))
+    assert solves('cuda:6', 5, True, um=one) == 1      # one structure waits in vain once
+    assert solves('cuda:6', 1, False) == 1             # and another one still tries
+    for _ in range(2):
+        assert solves('cuda:6', 3, True) == 3
+        assert solves('cuda:6', 1000, True) <= 5
+        assert solves('cuda:7', 4, False) == 4
+        assert solves('cuda:6', 5000, False) > 0       # the CUs are free again
+        assert solves('cuda:6', 10, False) == 10
+    assert solves('cuda:6', 2, True) == 2
+    assert solves('cuda:6', 3, False) == 3             # waits in a row count
