@@ -601,9 +601,29 @@ def test_device_pcg_against_reference_vectors(case, d, rtol):
         assert rel_err(x, xr) <= rtol
 
 
-def test_pcg_graph_replay_matches_eager():
+PCG_FORMS = ['rows', 'pairs', 'resident']
+
+
+def _force_pcg_form(monkeypatch, form):
+    """The solver's PCG by launches (products by row copies or by pair blocks), or resident where it applies."""
+    from blast3r_amd import ba_solver
+    if form != 'resident':
+        monkeypatch.setattr(GaussNewtonSolver, '_run_resident', lambda *a: False)
+        monkeypatch.setattr(ba_solver, 'PCG_ROWS_MOST', 0 if form == 'pairs' else 10 ** 12)
+
+
+def _check_pcg_form(gs, form):
+    ws = gs.last['plan']._ws
+    assert gs.last['pcg_resident'] == (form == 'resident')
+    assert ('pcg_S_rows' in ws) == (form == 'rows') and ('pcg_t' in ws) == (form == 'pairs')
+
+
+@pytest.mark.parametrize('form', PCG_FORMS)
+def test_pcg_graph_replay_matches_eager(form, monkeypatch):
     """The PCG replayed from its captured HIP graph equals the eager launches bit for bit on every
-    replay, with the program's own eager work and synchronisations between the replays."""
+    replay, with the program's own eager work and synchronisations between the replays; the resident
+    PCG, which has no graph, equals itself."""
+    _force_pcg_form(monkeypatch, form)
     p = make_problem(0, n_frames=12, n_tracks=600)
     g = _gpu(p)
     o = opts(p)
@@ -618,6 +638,7 @@ def test_pcg_graph_replay_matches_eager():
         J = gs.compute_jacobians(g.infos, g.K, g.P_rig2cam, g.P_w2rig, g.z_coefs, g.pts3d, g.pids, g.pix2d_std,
                                  g.pix2d_dep, True, pix2d=g.pix2d, hp=hp)
         d = gs.solve_delta(J, res, w)
+        _check_pcg_form(gs, form)
         return d.clone(), gs.last['istate'].clone()
 
     d_e, ist_e = solve(False)
@@ -1335,14 +1356,16 @@ def test_reduced_solve_cholesky_fallback_runs_pcg_and_points_again(cfg, nf, nt):
     assert torch.equal(deltas[0], deltas[1])
 
 
+@pytest.mark.parametrize('form', PCG_FORMS)
 @pytest.mark.parametrize('cfg,nf,nt,maxiter', [(0, None, None, 300), (2, 30, 1500, 300), (0, 16, 600, 60),
                                                 (0, 8, 300, 20)])
-def test_pcg_chunked_graphs_equal_the_whole_sequence(cfg, nf, nt, maxiter):
+def test_pcg_chunked_graphs_equal_the_whole_sequence(cfg, nf, nt, maxiter, form, monkeypatch):
     """The PCG replayed from chunk graphs, where the host stops launching chunks once the loop has stopped
-    (ba_pcg_solve_range, the flag read from pinned memory), gives the bits of the whole launch sequence
-    (ba_pcg_solve, use_graph off): delta and the loop's outcome equal, also on a second solve that replays the
+    (ba_pcg_solve_range and its form by pair blocks, the flag read from pinned memory), gives the bits of the whole
+    launch sequence (use_graph off): delta and the loop's outcome equal, also on a second solve that replays the
     captured graphs; where the loop converges early (full config 0) fewer iterations are launched, at most two
-    chunks past the stop."""
+    chunks past the stop.  The resident PCG, which has no graph, equals itself."""
+    _force_pcg_form(monkeypatch, form)
     from blast3r_amd.ba_solver import PCG_CHUNK
     print(f'pcg chunks cfg {cfg} ({nf} frames, {nt} tracks), maxiter {maxiter}', flush=True)
     p = make_problem(cfg, n_frames=nf, n_tracks=nt)
@@ -1362,6 +1385,7 @@ def test_pcg_chunked_graphs_equal_the_whole_sequence(cfg, nf, nt, maxiter):
                                  g.pix2d_dep, True, pix2d=g.pix2d, hp=hp, **flags)
         d1 = gs.solve_delta(J, res, w)
         d2 = gs.solve_delta(J, res, w)
+        _check_pcg_form(gs, form)
         runs[use_graph] = (d1, d2, gs.last['istate'].cpu(), gs.last['pcg_launched'])
     (c1, c2, c_ist, launched), (w1, w2, w_ist, _) = runs[True], runs[False]
     k, conv = int(w_ist[2]), int(w_ist[3])
@@ -1373,6 +1397,9 @@ def test_pcg_chunked_graphs_equal_the_whole_sequence(cfg, nf, nt, maxiter):
         assert launched <= k + 2 * PCG_CHUNK
     if cfg == 0 and nf is None:
         assert conv == 1 and launched < maxiter
+    if form != 'resident':
+        graphs = list(gs.last['plan']._pcg_graphs.values())
+        assert len(graphs) == 1 and graphs[0]['solves'] == 2 and (graphs[0]['chunks'] is not None) == (maxiter > PCG_CHUNK)
 
 
 _CHOL_CASES = [(0, 8, 300), (1, 32, 400), (2, 30, 1500), (3, 24, 600), (4, 20, 800), (2, 70, 3000)]
