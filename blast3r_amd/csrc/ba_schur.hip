@@ -1988,8 +1988,8 @@ static void pm_stage(const ba_pm_args& a, int stage, hipStream_t st) {
             // waves started, drained and joined for short ones cost more than they save, and where the pairs fill the
             // chip many times over only long ones gain.  Measured, a wave / a workgroup per pair, us: d = 11 fp64 at 56
             // terms a pair 47 / 46, 87: 203 / 226, 149: 184 / 170, 400: 124 / 107, 700: 530 / 464; fp32 at 84: 158 / 219,
-            // 112: 53 / 53, 520: 62 / 26; d > 15 (17, 23 and 25 alike) fp64 at 34: 61 / 59, 67: 104 / 88, 829: 1187 / 875; fp32
-            // at 34: 40 / 50, 67: 68 / 63, 829: 740 / 511; 820 pairs of 40: 10.3 / 8.4 (fp32 8.4 / 8.4), 36 of 118: 14.0 /
+            // 112: 53 / 53, 520: 62 / 26; d > 15 fp64 at 34: 61 / 59, 67: 104 / 88, 829: 1187 / 875 (d = 23 and 25; d = 17: 842);
+            // fp32 at 34: 40 / 50, 67: 68 / 63, 829: 740 / 511; 820 pairs of 40: 10.3 / 8.4 (fp32 8.4 / 8.4), 36 of 118: 14.0 /
             // 6.2; from 23 k pairs on: 543 k of 157: 7500 / 8240, 188 k of 227: 4180 / 4340, 27 k of 157: 490 / 494, 24 k of
             // 259: 680 / 657, d > 15 24 k of 259: 1400 / 1340 (fp32 790 / 733), of 130: fp64 715 / 700, fp32 385 / 413, 27 k
             // of 62: 438 / 488, 53 k of 77: 944 / 1034 (fp32 518 / 643), of 39: 484 / 623 (289 / 521)
