@@ -1004,16 +1004,9 @@ __global__ void __launch_bounds__(PP_T) k_pcg_resident(ba_pcg_args a, ba_pcg_res
         if (k < wave) base += sCnt[k];
         ncol += sCnt[k];
     }
-    // blocks of the longest row per lane group, and the blocks that go to LDS; sizes of a plan for other rows or another
-    // m would let them and the columns run past their arrays: the solve is given up then, by all threads alike
-    const int gpr = NG / m;                                             // lane groups per row
-    int nbr = 0, nlds = 0;
-    for (int q = i0; q < i1; ++q) {                                     // at most 32 rows
-        const int len = a.row_ptr[q + 1] - a.row_ptr[q];
-        nbr = max(nbr, (len + gpr - 1) / gpr);
-        nlds += max(0, len - NBR * gpr);
-    }
-    if (ncol > w.max_col || nlds > w.max_blk) {
+    // max_col or max_blk of a plan for other rows or another m: the columns or (below) the LDS blocks would run past their
+    // arrays; the solve is given up, by all threads alike
+    if (__builtin_expect(ncol > w.max_col, 0)) {
         if (tid == 0) a.istate[6] = 1;
         return;
     }
@@ -1026,6 +1019,7 @@ __global__ void __launch_bounds__(PP_T) k_pcg_resident(ba_pcg_args a, ba_pcg_res
     int u[PP_E], sh[PP_E], oy[PP_E], op[PP_E], ow[PP_E];
     bool counts[PP_E];
     Real x[PP_E], xb_[PP_E], r[PP_E], z[PP_E], p[PP_E], dA[PP_E], iA[PP_E], dmp[PP_E];
+    const int gpr = NG / m;                                             // lane groups per row
 #pragma unroll
     for (int k = 0; k < PP_E; ++k) {
         const int e = lane + 64 * k, el = e / d, ej = e - el * d;
@@ -1073,12 +1067,16 @@ __global__ void __launch_bounds__(PP_T) k_pcg_resident(ba_pcg_args a, ba_pcg_res
     int bx[NBR + 1];                                                        // the column slots of the register blocks
     {
         int at = 0;
-        for (int q = 0; q < i1 - i0; ++q) {                             // rows in order
+        for (int q = 0; q < i1 - i0; ++q) {                             // rows in order: at most 32
             const int b0 = a.row_ptr[i0 + q] - e0, len = a.row_ptr[i0 + q + 1] - e0 - b0;
             const int more = max(0, len - NBR * gpr);
+            if (__builtin_expect(at + more > w.max_blk, 0)) {
+                if (tid == 0) a.istate[6] = 1;
+                return;
+            }
             for (int t = tid; t < more; t += PP_T) sCidx[at + t] = map[col_of(b0 + NBR * gpr + t)] * GW;
             if (q == row) { ls0 = at; ls1 = at + more; }
-            at += more;                                                 // at most max_blk
+            at += more;
         }
     }
     const int rb0 = row < i1 - i0 ? a.row_ptr[i0 + row] - e0 : 0, rb1 = row < i1 - i0 ? a.row_ptr[i0 + row + 1] - e0 : 0;
@@ -1093,6 +1091,8 @@ __global__ void __launch_bounds__(PP_T) k_pcg_resident(ba_pcg_args a, ba_pcg_res
         for (int c = 0; c < DM; ++c)
             B[k][c] = live && j < d && c < d ? ((ent & 1) ? S[c * d + j] : S[j * d + c]) : Real(0);
     }
+    int nbr = 0;                                                        // register blocks of the longest row
+    for (int q = 0; q < i1 - i0; ++q) nbr = max(nbr, (a.row_ptr[i0 + q + 1] - a.row_ptr[i0 + q] + gpr - 1) / gpr);
     __syncthreads();                                                    // the map is done with
     {
         int at = 0;
